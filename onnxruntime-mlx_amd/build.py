@@ -24,7 +24,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
 KERNEL_SOURCES = ["runtime.hip", "mnb.hip", "mnb_blk.hip", "mnb_gemm.hip", "attention.hip",
-                  "norm.hip", "decode_step.hip", "gqa_ext.hip"]
+                  "attn_tile.hip", "norm.hip", "decode_step.hip", "gqa_ext.hip"]
 EP_SOURCES = ["ep/ep.cpp", "ep/graph.cpp", "ep/fuse.cpp", "ep/plan.cpp"]
 
 HIP_FLAGS = [

@@ -1,6 +1,8 @@
 // GroupQueryAttention, PagedAttention and RotaryEmbedding for gfx950.
 //
 // Kernels:
+//  * gqa_kv_rows - new rows in 16-byte pieces, where rotary dims fill the head
+//    and tensors are aligned; the prep kernel below takes the rest.
 //  * gqa_prep / paged_prep - per new token: optional QK RMS-norm, RoPE on Q and K
 //    (fp32 math, one rounding to the op dtype), new K/V written to their cache
 //    rows (dense present buffer or paged slot); rotated Q (and, paged, rotated K)
@@ -12,17 +14,17 @@
 //    contiguous rows per load), and in the growing contract writes the same rows
 //    to `present` from the registers it already holds, so the past->present copy
 //    costs no extra read. Partial softmax states are merged by attn_merge.
-//  * gqa_tile / paged_tile - matrix-core flash-attention tiles for everything
-//    with more than one query token (GQA prefill, PagedAttention prefill
-//    chunks): S^T = K.Q^T and O^T += V^T.P^T on v_mfma_f32_32x32x16_f16, Q^T
-//    and K staged in LDS, V transposed in LDS, online softmax in fp32 with one
-//    query per lane. Paged keys are fetched through the block table on the
-//    device; no control tensor is read back to the host.
+//  * paged_tile - matrix-core flash-attention tiles for PagedAttention's prefill chunks
+//    (GroupQueryAttention's prompts: attn_tile.hip): S^T = K.Q^T and O^T += V^T.P^T on
+//    v_mfma_f32_32x32x16_f16, Q^T and K staged in LDS, V transposed in LDS, online
+//    softmax in fp32 with one query per lane. Paged keys are fetched through the block
+//    table on the device; no control tensor is read back to the host.
 //  * paged_decode - one-token PagedAttention rows on the vector units, split-K.
 //  * attn_merge / paged_merge - log-sum-exp merge of split-K partials.
 #include <mutex>
 #include <type_traits>
 
+#include "attn_internal.h"
 #include "common.h"
 
 namespace ortmi {
@@ -158,6 +160,95 @@ __global__ __launch_bounds__(64 * kPrepHeads) void gqa_prep_kernel(
         lds_to_row<T>(pk + row, sv, hd, lane);
         copy_row<T>(pv + row, v + (int64_t)tok * kv_stride + (int64_t)kvh * hd, hd, lane);
     }
+}
+
+// The new rows alone, in 16-byte pieces, where the tile kernel rotates the queries as it
+// loads them: one thread takes the 8 dims from 8c and the 8 from hd/2 + 8c of a (token,
+// KV head), K rotated (rotary dims = hd; cos null: as it is) and V copied to present rows
+// vp + s. Bound by its 16-byte accesses; 2048 tokens of 32 + 8 heads of 128, whose rotated
+// queries went through memory as well: 22 us before.
+template <typename T>
+__device__ __forceinline__ void unpack8(u32x4_t w, float (&x)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        x[2 * i] = to_f32(__builtin_bit_cast(T, (uint16_t)(w[i] & 0xffffu)));
+        x[2 * i + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(w[i] >> 16)));
+    }
+}
+template <typename T>
+__device__ __forceinline__ u32x4_t pack8(const float (&x)[8]) {
+    u32x4_t w;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        w[i] = (uint32_t)__builtin_bit_cast(uint16_t, from_f32<T>(x[2 * i])) |
+               (uint32_t)__builtin_bit_cast(uint16_t, from_f32<T>(x[2 * i + 1])) << 16;
+    return w;
+}
+// Rotates the pieces w0 (dims c .. c + 7) and w1 (dims hd/2 + c ..) of a head whose rotary
+// dims fill it (half = hd / 2), one rounding to T.
+template <typename T>
+__device__ __forceinline__ void rope_pieces(u32x4_t& w0, u32x4_t& w1, const T* cos_row,
+                                            const T* sin_row, int c, int half, int interleaved) {
+    float x[8], y[8], cs[8], sn[8];
+    unpack8<T>(w0, x);
+    unpack8<T>(w1, y);
+    if (interleaved) {
+        // Pairs (2i, 2i + 1) inside a piece: entries c/2.. and half/2 + c/2.. .
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            cs[j] = to_f32(cos_row[c / 2 + j]);
+            sn[j] = to_f32(sin_row[c / 2 + j]);
+            cs[4 + j] = to_f32(cos_row[half / 2 + c / 2 + j]);
+            sn[4 + j] = to_f32(sin_row[half / 2 + c / 2 + j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float a = x[2 * j], d = x[2 * j + 1], e = y[2 * j], f = y[2 * j + 1];
+            x[2 * j] = a * cs[j] - d * sn[j];
+            x[2 * j + 1] = d * cs[j] + a * sn[j];
+            y[2 * j] = e * cs[4 + j] - f * sn[4 + j];
+            y[2 * j + 1] = f * cs[4 + j] + e * sn[4 + j];
+        }
+    } else {
+        unpack8<T>(*reinterpret_cast<const u32x4_t*>(cos_row + c), cs);
+        unpack8<T>(*reinterpret_cast<const u32x4_t*>(sin_row + c), sn);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float a = x[j], d = y[j];
+            x[j] = a * cs[j] - d * sn[j];
+            y[j] = d * cs[j] + a * sn[j];
+        }
+    }
+    w0 = pack8<T>(x);
+    w1 = pack8<T>(y);
+}
+template <typename T>
+__global__ __launch_bounds__(256) void gqa_kv_rows_kernel(
+    const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ cos_c,
+    const T* __restrict__ sin_c, int interleaved, T* __restrict__ pk, T* __restrict__ pv, int S,
+    int KV, int hd, int64_t pcap, int vp, int64_t kv_stride, int64_t items) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= items) return;
+    const int pieces = hd / 16, half = hd / 2;
+    const int c = (int)(i % pieces) * 8;
+    const int64_t th = i / pieces;
+    const int kvh = (int)(th % KV);
+    const int64_t tok = th / KV;
+    const int s = (int)(tok % S);
+    const int64_t b = tok / S;
+    const int64_t src = tok * kv_stride + (int64_t)kvh * hd + c;
+    const int64_t dst = ((b * KV + kvh) * pcap + vp + s) * hd + c;
+    auto load = [](const T* p) { return *reinterpret_cast<const u32x4_t*>(p); };
+    auto store = [](T* p, u32x4_t w) { *reinterpret_cast<u32x4_t*>(p) = w; };
+    u32x4_t k0 = load(k + src), k1 = load(k + src + half);
+    store(pv + dst, load(v + src));
+    store(pv + dst + half, load(v + src + half));
+    if (cos_c) {
+        const int64_t crow = (int64_t)(vp + s) * half;
+        rope_pieces<T>(k0, k1, cos_c + crow, sin_c + crow, c, half, interleaved);
+    }
+    store(pk + dst, k0);
+    store(pk + dst + half, k1);
 }
 
 __global__ __launch_bounds__(256) void kv_copy_kernel(const uint4* __restrict__ src,
@@ -609,8 +700,10 @@ __global__ __launch_bounds__(256) void gqa_decode_kernel(
 // cases compute the split weights once into LDS, then each thread sums its
 // output dims over the splits.
 constexpr int kMergeFast = 16;
-// Most key splits of a dense prefill tile (each split writes a partial row).
-constexpr int kPrefillSplits = 2;
+// Key splits of a dense prefill tile (each writes a partial row): the workspace has room
+// for two at least, and for up to 16 where few rows would leave CUs idle (a tile has up
+// to 128 rows, the chip 256 CUs).
+constexpr int kPrefillSplits = 2, kMaxPrefillSplits = kMergeFast;
 template <typename T>
 __global__ __launch_bounds__(128) void attn_merge_kernel(const float* __restrict__ part,
                                                          T* __restrict__ out, int nsplit,
@@ -691,14 +784,6 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(const float* __restrict
 
 // ------------------------------------------------------------ attn_tile --
 
-// Key/value source for one (sequence, kv head).
-struct DenseKV {
-    // [B, KV, cap, hd]
-    const void* k;
-    const void* v;
-    int64_t cap;
-    int KV;
-};
 struct PagedKV {
     const void* kcache;  // [nblk, blk, KV, hd]
     const void* vcache;  // [nblk, blk, KV, vhd] or null (latent)
@@ -721,174 +806,7 @@ struct TileDesc {
     int tok_seq0;   // first packed token of the sequence (paged)
 };
 
-constexpr int kTileRows = 64;   // max query rows per workgroup
 constexpr int kKeyTile = 64;
-
-template <typename T, int HD, int VHD, bool PAGED>
-__device__ __forceinline__ const T* key_ptr(const DenseKV& d, const PagedKV& p, const TileDesc& t,
-                                            int b, int kvh, int j, bool value) {
-    if constexpr (!PAGED) {
-        const T* base = static_cast<const T*>(value ? d.v : d.k);
-        return base + (((int64_t)b * d.KV + kvh) * d.cap + j) * (value ? VHD : HD);
-    } else {
-        if (j >= t.past) {
-            const int tok = t.tok_seq0 + (j - t.past);
-            if (value && p.vnew)
-                return static_cast<const T*>(p.vnew) + ((int64_t)tok * p.KV + kvh) * VHD;
-            return static_cast<const T*>(p.knew) + ((int64_t)tok * p.KV + kvh) * HD;
-        }
-        const int lb = j / p.blk;
-        const int phys = (j >= 0 && lb < p.maxb) ? p.bt[(int64_t)t.seq * p.maxb + lb] : -1;
-        if (phys < 0 || phys >= p.nblk) return nullptr;
-        const int64_t slot = (int64_t)phys * p.blk + (j % p.blk);
-        if (value && p.vcache)
-            return static_cast<const T*>(p.vcache) + (slot * p.KV + kvh) * VHD;
-        return static_cast<const T*>(p.kcache) + (slot * p.KV + kvh) * HD;
-    }
-}
-
-// One workgroup: `rows` = ntok * G query rows (row r -> token r / G, head r % G
-// of the group) against keys [k0, k1) of one (sequence, kv head). When
-// `part` is null the normalised output is written; otherwise the partial state.
-template <typename T, int HD, int VHD, bool PAGED>
-__device__ void attn_tile_body(const TileDesc& t, int kvh, int G, int H, const T* __restrict__ qrot,
-                               const DenseKV& dk, const PagedKV& pk, float scale,
-                               const float* __restrict__ sink, int k0, int k1,
-                               T* __restrict__ out, int64_t out_tok_stride,
-                               float* __restrict__ part, int nsplit, int split) {
-    __shared__ float sQ[kTileRows][HD + 1];
-    __shared__ T sK[kKeyTile][HD + 8];
-    __shared__ T sV[kKeyTile][VHD + 8];
-    __shared__ float sS[kTileRows][kKeyTile + 1];
-    __shared__ float sM[kTileRows], sL[kTileRows], sAlpha[kTileRows];
-    __shared__ int sOk[kKeyTile];
-
-    const int tid = threadIdx.x;
-    const int rows = t.ntok * G;
-    for (int idx = tid; idx < kTileRows * HD; idx += 256) {
-        const int r = idx / HD, d = idx % HD;
-        float v = 0.f;
-        if (r < rows) {
-            const int tok = t.tok0 + r / G, h = kvh * G + r % G;
-            v = to_f32(qrot[((int64_t)tok * H + h) * HD + d]) * scale;
-        }
-        sQ[r][d] = v;
-    }
-    if (tid < kTileRows) {
-        sM[tid] = -INFINITY;
-        sL[tid] = 0.f;
-    }
-    // Thread -> (row, 16-key slice) for scores; (row, VHD/4 dims) for P.V.
-    const int r_s = tid / 4, c_s = (tid % 4) * 16;
-    constexpr int DV = VHD / 4;
-    const int d_o = (tid % 4) * DV;
-    float o[DV];
-#pragma unroll
-    for (int i = 0; i < DV; ++i) o[i] = 0.f;
-    const bool row_live = r_s < rows;
-    const int qpos = t.qpos0 + r_s / G;
-    __syncthreads();
-
-    for (int kb = k0; kb < k1; kb += kKeyTile) {
-        const int nk = min(kKeyTile, k1 - kb);
-        // Stage K/V tile (16-byte vectors).
-        constexpr int KV_VEC = HD / 8, VV_VEC = VHD / 8;
-        for (int idx = tid; idx < kKeyTile * KV_VEC; idx += 256) {
-            const int r = idx / KV_VEC, c = (idx % KV_VEC) * 8;
-            uint4 val = make_uint4(0, 0, 0, 0);
-            const T* p = r < nk ? key_ptr<T, HD, VHD, PAGED>(dk, pk, t, t.seq, kvh, kb + r, false)
-                                : nullptr;
-            if (p) val = *reinterpret_cast<const uint4*>(p + c);
-            *reinterpret_cast<uint4*>(&sK[r][c]) = val;
-            if (c == 0) sOk[r] = p != nullptr;
-        }
-        for (int idx = tid; idx < kKeyTile * VV_VEC; idx += 256) {
-            const int r = idx / VV_VEC, c = (idx % VV_VEC) * 8;
-            uint4 val = make_uint4(0, 0, 0, 0);
-            if (r < nk) {
-                const T* p = key_ptr<T, HD, VHD, PAGED>(dk, pk, t, t.seq, kvh, kb + r, true);
-                if (p) val = *reinterpret_cast<const uint4*>(p + c);
-            }
-            *reinterpret_cast<uint4*>(&sV[r][c]) = val;
-        }
-        __syncthreads();
-        // Scores.
-        float tmax = -INFINITY;
-        if (row_live) {
-            for (int c = 0; c < 16; ++c) {
-                const int jj = c_s + c, j = kb + jj;
-                float sc = -INFINITY;
-                const bool ok = jj < nk && j <= qpos && sOk[jj];
-                if (ok) {
-                    float acc = 0.f;
-#pragma unroll 16
-                    for (int d = 0; d < HD; ++d) acc = fmaf(sQ[r_s][d], to_f32(sK[jj][d]), acc);
-                    sc = acc;
-                }
-                sS[r_s][jj] = sc;
-                tmax = fmaxf(tmax, sc);
-            }
-        }
-        tmax = group_max<4>(tmax);
-        __syncthreads();
-        if (row_live) {
-            const float m_old = sM[r_s];
-            const float m_new = fmaxf(m_old, tmax);
-            float lsum = 0.f;
-            for (int c = 0; c < 16; ++c) {
-                const int jj = c_s + c;
-                const float e = (m_new == -INFINITY) ? 0.f : __expf(sS[r_s][jj] - m_new);
-                sS[r_s][jj] = e;
-                lsum += e;
-            }
-            lsum = group_sum<4>(lsum);  // the 4 lanes of a row share row_live
-            const float alpha = (m_old == -INFINITY) ? 0.f : __expf(m_old - m_new);
-            if ((tid % 4) == 0) {
-                sL[r_s] = sL[r_s] * alpha + lsum;
-                sM[r_s] = m_new;
-                sAlpha[r_s] = alpha;
-            }
-        }
-        __syncthreads();
-        if (row_live) {
-            const float alpha = sAlpha[r_s];
-#pragma unroll
-            for (int i = 0; i < DV; ++i) o[i] *= alpha;
-            for (int jj = 0; jj < nk; ++jj) {
-                const float p = sS[r_s][jj];
-#pragma unroll
-                for (int i = 0; i < DV; ++i) o[i] = fmaf(p, to_f32(sV[jj][d_o + i]), o[i]);
-            }
-        }
-        __syncthreads();
-    }
-    if (!row_live) return;
-    const int tok = t.tok0 + r_s / G, h = kvh * G + r_s % G;
-    float m = sM[r_s], l = sL[r_s];
-    if (part) {
-        // Partial rows are token-major: row tok * H + h.
-        float* dst = part + (((int64_t)tok * H + h) * nsplit + split) * (VHD + 2);
-#pragma unroll
-        for (int i = 0; i < DV; ++i) dst[d_o + i] = o[i];
-        if ((tid % 4) == 0) {
-            dst[VHD] = m;
-            dst[VHD + 1] = l;
-        }
-        return;
-    }
-    if (sink) {
-        const float sv = sink[h];
-        const float mm = fmaxf(m, sv);
-        const float a = (m == -INFINITY) ? 0.f : __expf(m - mm);
-        l = l * a + __expf(sv - mm);
-#pragma unroll
-        for (int i = 0; i < DV; ++i) o[i] *= a;
-    }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
-    T* dst = out + (int64_t)tok * out_tok_stride + (int64_t)h * VHD + d_o;
-#pragma unroll
-    for (int i = 0; i < DV; ++i) dst[i] = from_f32<T>(o[i] * inv);
-}
 
 // The attention tile on the matrix cores (fp16), 128 query rows per workgroup,
 // computed transposed so that everything a query needs stays in its lanes:
@@ -941,10 +859,9 @@ __device__ __forceinline__ float tile_pair_sum(uint32_t w, float acc) {
     }
 }
 
-template <typename T, int HD, int VHD, bool PAGED, int NW = 4>
+template <typename T, int HD, int VHD, int NW>
 __device__ void attn_mfma_body(const TileDesc& t, int kvh, int G, int H,
-                               const T* __restrict__ qrot, const DenseKV& dk,
-                               const PagedKV& pk, float scale, const float* __restrict__ sink,
+                               const T* __restrict__ qrot, const PagedKV& pk, float scale, const float* __restrict__ sink,
                                int k0, int k1, T* __restrict__ out, int64_t out_tok_stride,
                                float* __restrict__ part, int nsplit, int split) {
     static_assert(std::is_same<T, half_t>::value || std::is_same<T, uint16_t>::value,
@@ -1015,26 +932,24 @@ __device__ void attn_mfma_body(const TileDesc& t, int kvh, int G, int H,
     // or more, reads the table from global memory instead (the second form of the
     // walk below).
     constexpr int kBtLds = 512;
-    __shared__ uint32_t s_bt[PAGED ? kBtLds : 1];
+    __shared__ uint32_t s_bt[kBtLds];
     int lb0 = 0;
     bool bt_lds = true;
-    if constexpr (PAGED) {
-        const int cend = min(k1, t.past);
-        if (cend > k0) {
-            lb0 = k0 / pk.blk;
-            const int n = (cend - 1) / pk.blk - lb0 + 1;
-            bt_lds = n <= kBtLds && pk.nblk * pk.blk * pk.KV < (int64_t)0xffffffff;
-            if (bt_lds)
-                for (int i = tid; i < n; i += NT) {
-                    const int lb = lb0 + i;
-                    const int phys = lb < pk.maxb ? pk.bt[(int64_t)t.seq * pk.maxb + lb] : -1;
-                    s_bt[i] = phys >= 0 && phys < pk.nblk
-                                  ? ((uint32_t)phys * (uint32_t)pk.blk) * (uint32_t)pk.KV + kvh
-                                  : ~0u;
-                }
-        }
-        __syncthreads();
+    const int cend = min(k1, t.past);
+    if (cend > k0) {
+        lb0 = k0 / pk.blk;
+        const int n = (cend - 1) / pk.blk - lb0 + 1;
+        bt_lds = n <= kBtLds && pk.nblk * pk.blk * pk.KV < (int64_t)0xffffffff;
+        if (bt_lds)
+            for (int i = tid; i < n; i += NT) {
+                const int lb = lb0 + i;
+                const int phys = lb < pk.maxb ? pk.bt[(int64_t)t.seq * pk.maxb + lb] : -1;
+                s_bt[i] = phys >= 0 && phys < pk.nblk
+                              ? ((uint32_t)phys * (uint32_t)pk.blk) * (uint32_t)pk.KV + kvh
+                              : ~0u;
+            }
     }
+    __syncthreads();
     // Byte address of new row 0 of the sequence's (virtual) new-row range, such
     // that key j >= past is at nrow0 + j * nstride (modular arithmetic).
     // Cache and new rows, keys and values alike, are HD dims apart: with a value
@@ -1055,42 +970,36 @@ __device__ void attn_mfma_body(const TileDesc& t, int kvh, int G, int H,
     // make the wait for its table entry wait for the K/V loads issued before it
     // (loads retire in order), and the block's loads would run one at a time.
     auto row_src = [&](int j, bool value, bool& ok, auto lds) -> const half_t* {
-        if constexpr (!PAGED) {
-            ok = true;
-            const half_t* base = static_cast<const half_t*>(value ? dk.v : dk.k);
-            return base + (((int64_t)t.seq * dk.KV + kvh) * dk.cap + j) * (value ? VHD : HD);
+        const bool fresh = j >= t.past;
+        const int jc = fresh ? k0 : j;  // a cache row stands in for a new one
+        int lb, within;
+        if (pk.blk_shift >= 0) {
+            lb = jc >> pk.blk_shift;
+            within = jc & ((1 << pk.blk_shift) - 1);
         } else {
-            const bool fresh = j >= t.past;
-            const int jc = fresh ? k0 : j;  // a cache row stands in for a new one
-            int lb, within;
-            if (pk.blk_shift >= 0) {
-                lb = jc >> pk.blk_shift;
-                within = jc & ((1 << pk.blk_shift) - 1);
-            } else {
-                lb = jc / pk.blk;
-                within = jc - lb * pk.blk;
-            }
-            const char* ac;
-            bool cok;
-            if constexpr (decltype(lds)::value) {
-                const uint32_t e = s_bt[min((unsigned)(lb - lb0), (unsigned)(kBtLds - 1))];
-                cok = e != ~0u;
-                const uint32_t r = (cok ? e : 0u) + __umul24((uint32_t)within, (uint32_t)pk.KV);
-                const char* cb = static_cast<const char*>((value && pk.vcache) ? pk.vcache : pk.kcache);
-                ac = cb + (uint64_t)r * kRowBytes;
-            } else {
-                // maxb >= 1 (the entry point checks it), so the clamped index is in range.
-                const int e = pk.bt[(int64_t)t.seq * pk.maxb + min(lb, pk.maxb - 1)];
-                const int phys = lb < pk.maxb ? e : -1;
-                cok = phys >= 0 && phys < pk.nblk;
-                const int64_t slot = (int64_t)(cok ? phys : 0) * pk.blk + within;
-                const char* cb = static_cast<const char*>((value && pk.vcache) ? pk.vcache : pk.kcache);
-                ac = cb + (uint64_t)(slot * pk.KV + kvh) * kRowBytes;
-            }
-            const char* an = (value ? nrow_v : nrow_k) + (uint64_t)(uint32_t)j * (uint64_t)nstride;
-            ok = fresh || cok;
-            return reinterpret_cast<const half_t*>(fresh ? an : ac);
+            lb = jc / pk.blk;
+            within = jc - lb * pk.blk;
         }
+        const char* ac;
+        bool cok;
+        if constexpr (decltype(lds)::value) {
+            const uint32_t e = s_bt[min((unsigned)(lb - lb0), (unsigned)(kBtLds - 1))];
+            cok = e != ~0u;
+            const uint32_t r = (cok ? e : 0u) + __umul24((uint32_t)within, (uint32_t)pk.KV);
+            const char* cb = static_cast<const char*>((value && pk.vcache) ? pk.vcache : pk.kcache);
+            ac = cb + (uint64_t)r * kRowBytes;
+        } else {
+            // maxb >= 1 (the entry point checks it), so the clamped index is in range.
+            const int e = pk.bt[(int64_t)t.seq * pk.maxb + min(lb, pk.maxb - 1)];
+            const int phys = lb < pk.maxb ? e : -1;
+            cok = phys >= 0 && phys < pk.nblk;
+            const int64_t slot = (int64_t)(cok ? phys : 0) * pk.blk + within;
+            const char* cb = static_cast<const char*>((value && pk.vcache) ? pk.vcache : pk.kcache);
+            ac = cb + (uint64_t)(slot * pk.KV + kvh) * kRowBytes;
+        }
+        const char* an = (value ? nrow_v : nrow_k) + (uint64_t)(uint32_t)j * (uint64_t)nstride;
+        ok = fresh || cok;
+        return reinterpret_cast<const half_t*>(fresh ? an : ac);
     };
     // A 64-key block into registers, keys and values separately: the row addresses
     // first, then the loads back to back. Loads are never conditional (a branch
@@ -1328,86 +1237,6 @@ __device__ void attn_mfma_body(const TileDesc& t, int kvh, int G, int H,
         }
 }
 
-// Tile body for a dtype: the matrix-core tile for fp16 and bf16 (NW waves of 32
-// query rows), the VALU tile (kTileRows rows, 256 threads) otherwise.
-template <typename T, int VHD>
-constexpr bool mfma_tile() {
-    return (std::is_same<T, half_t>::value || std::is_same<T, uint16_t>::value) && VHD % 32 == 0;
-}
-// Query rows per workgroup of the tile body used for dtype T.
-template <typename T>
-static int tile_rows_for(int vhd, int nw = 4) {
-    return (std::is_same<T, half_t>::value || std::is_same<T, uint16_t>::value) && vhd % 32 == 0
-               ? 32 * nw
-               : kTileRows;
-}
-// Threads of a tile workgroup.
-template <typename T, int VHD, int NW>
-constexpr int tile_threads() {
-    return mfma_tile<T, VHD>() ? 64 * NW : 256;
-}
-
-template <typename T, int HD, int VHD, bool PAGED, int NW = 4>
-__device__ __forceinline__ void attn_tile(const TileDesc& t, int kvh, int G, int H,
-                                          const T* __restrict__ qrot, const DenseKV& dk,
-                                          const PagedKV& pk, float scale,
-                                          const float* __restrict__ sink, int k0, int k1,
-                                          T* __restrict__ out, int64_t out_tok_stride,
-                                          float* __restrict__ part, int nsplit, int split) {
-    if constexpr (mfma_tile<T, VHD>())
-        attn_mfma_body<T, HD, VHD, PAGED, NW>(t, kvh, G, H, qrot, dk, pk, scale, sink, k0, k1, out,
-                                            out_tok_stride, part, nsplit, split);
-    else
-        attn_tile_body<T, HD, VHD, PAGED>(t, kvh, G, H, qrot, dk, pk, scale, sink, k0, k1, out,
-                                          out_tok_stride, part, nsplit, split);
-}
-
-// GQA prefill / S > 1: grid (B * tiles_per_seq, KV). Keys from `present`. The
-// matrix-core tile takes 8 waves (256 query rows, one workgroup per CU), as the
-// paged tile does: the per-thread K/V prefetch halves, which keeps the body
-// within 256 VGPRs.
-constexpr int kGqaTileWaves = 8;
-template <typename T, int HD>
-__global__ __launch_bounds__((tile_threads<T, HD, kGqaTileWaves>()),
-                             (mfma_tile<T, HD>() ? 1 : 2)) void gqa_tile_kernel(const T* __restrict__ qrot, DenseKV dk,
-                                                       int S, int QT, int tiles_per_seq, int G,
-                                                       int H, int vp, float scale,
-                                                       T* __restrict__ out, int chunk, int nsplit,
-                                                       float* __restrict__ part,
-                                                       int* __restrict__ nsplit_row) {
-    const int b = blockIdx.x / tiles_per_seq;
-    const int tile = blockIdx.x % tiles_per_seq;
-    const int kvh = blockIdx.y, split = blockIdx.z;
-    TileDesc t;
-    t.seq = b;
-    const int s0 = tile * QT;
-    t.ntok = min(QT, S - s0);
-    t.tok0 = b * S + s0;
-    t.qpos0 = vp + s0;
-    t.past = vp;
-    t.nkeys = vp + S;
-    t.tok_seq0 = b * S;
-    PagedKV none{};
-    const int k1 = min(t.nkeys, t.qpos0 + t.ntok);  // causal bound of the tile
-    // Key splits of `chunk` keys (the last takes the rest); rows of a tile that
-    // needs one split are written directly and marked 0 for the merge.
-    const int ns = min(nsplit, max(1, (k1 + chunk - 1) / chunk));
-    if (split == 0 && nsplit > 1) {
-        for (int r = threadIdx.x; r < t.ntok * G; r += blockDim.x)
-            nsplit_row[(int64_t)(t.tok0 + r / G) * H + kvh * G + r % G] = ns > 1 ? ns : 0;
-    }
-    if (split >= ns) return;
-    if (ns == 1) {
-        attn_tile<T, HD, HD, false, kGqaTileWaves>(t, kvh, G, H, qrot, dk, none, scale, nullptr,
-                                                   0, k1, out, (int64_t)H * HD, nullptr, 1, 0);
-        return;
-    }
-    const int k0 = split * chunk;
-    const int ks1 = split == ns - 1 ? k1 : min(k1, k0 + chunk);
-    attn_tile<T, HD, HD, false, kGqaTileWaves>(t, kvh, G, H, qrot, dk, none, scale, nullptr, k0,
-                                               ks1, out, (int64_t)H * HD, part, nsplit, split);
-}
-
 // ------------------------------------------------------- PagedAttention --
 
 // Tile map built on the device by one 64-lane wave (no host read of the control
@@ -1545,8 +1374,7 @@ __global__ __launch_bounds__(64 * kPrepHeads) void paged_prep_kernel(
 // K/V block fetched serves twice the queries of a 4-wave tile.
 constexpr int kPagedTileWaves = 8;
 template <typename T, int HD, int VHD>
-__global__ __launch_bounds__((tile_threads<T, VHD, kPagedTileWaves>()),
-                             (mfma_tile<T, VHD>() ? 1 : 2)) void paged_tile_kernel(
+__global__ __launch_bounds__(64 * kPagedTileWaves, 1) void paged_tile_kernel(
     const int4* __restrict__ tiles, const int* __restrict__ tile_count,
     const int32_t* __restrict__ cum, const int32_t* __restrict__ past_lens, PagedKV pk,
     const T* __restrict__ qrot, int G, int H, float scale, const float* __restrict__ sink,
@@ -1575,7 +1403,6 @@ __global__ __launch_bounds__((tile_threads<T, VHD, kPagedTileWaves>()),
     t.qpos0 = t.past + (t.tok0 - t.tok_seq0);
     t.nkeys = t.qpos0 + t.ntok;
     const int kend = min(t.nkeys, pk.max_ctx);  // causal bound of the tile
-    DenseKV none{};
     const int ns = min(nsplit, max(1, (kend + chunk - 1) / chunk));
     if (split == 0) {
         for (int r = threadIdx.x; r < t.ntok * G; r += blockDim.x)
@@ -1583,13 +1410,13 @@ __global__ __launch_bounds__((tile_threads<T, VHD, kPagedTileWaves>()),
     }
     if (split >= ns) return;
     if (ns == 1) {
-        attn_tile<T, HD, VHD, true, kPagedTileWaves>(t, kvh, G, H, qrot, none, pk, scale, sink, 0, kend, out,
+        attn_mfma_body<T, HD, VHD, kPagedTileWaves>(t, kvh, G, H, qrot, pk, scale, sink, 0, kend, out,
                                     (int64_t)H * VHD, nullptr, 1, 0);
         return;
     }
     const int k0 = split * chunk;
     const int k1 = split == ns - 1 ? kend : min(kend, k0 + chunk);
-    attn_tile<T, HD, VHD, true, kPagedTileWaves>(t, kvh, G, H, qrot, none, pk, scale, sink, k0, k1, out,
+    attn_mfma_body<T, HD, VHD, kPagedTileWaves>(t, kvh, G, H, qrot, pk, scale, sink, k0, k1, out,
                                 (int64_t)H * VHD, part, nsplit, split);
 }
 
@@ -1977,11 +1804,11 @@ using namespace ortmi;
 
 // ---------------------------------------------------------------- GQA API --
 
-extern "C" size_t ortmi_group_query_attention_workspace_size(int64_t batch, int64_t seq_len,
-                                                             int64_t num_heads, int64_t head_size,
-                                                             int64_t total_kv) {
-    // qrot (fp32-sized upper bound) + decode partials, or the prefill tiles' split
-    // partials and per-row split counts.
+namespace ortmi {
+// qrot (fp32-sized upper bound) + decode partials, or the prefill tiles' per-row split
+// counts and the partials of `splits` splits.
+static size_t gqa_workspace(int64_t batch, int64_t seq_len, int64_t num_heads, int64_t head_size,
+                            int64_t total_kv, int64_t splits) {
     size_t q = align_up((size_t)batch * seq_len * num_heads * head_size * 4);
     // Chunks are at least 64 keys, so ceil(total_kv / 64) bounds the split count.
     const int64_t nkv = total_kv > 0 ? total_kv : 1;
@@ -1989,14 +1816,28 @@ extern "C" size_t ortmi_group_query_attention_workspace_size(int64_t batch, int6
     size_t part = align_up((size_t)batch * num_heads * (size_t)ns * (head_size + 2) * 4);
     if (seq_len > 1) {
         const size_t rows = (size_t)batch * seq_len * num_heads;
-        part = std::max(part, align_up(rows * kPrefillSplits * (head_size + 2) * 4) +
+        part = std::max(part, align_up(rows * (size_t)splits * (head_size + 2) * 4) +
                                   align_up(rows * 4));
     }
-    // Head 96 takes the generic kernels for everything but the one-token decode.
+    // Head 96 takes the generic kernels for the decode steps and tensors that the others
+    // do not take.
     if (head_size == 96)
         return std::max(q + part, ortmi_group_query_attention_ex_workspace_size(
                                       batch, seq_len, num_heads, head_size));
     return q + part;
+}
+}  // namespace ortmi
+
+extern "C" size_t ortmi_group_query_attention_workspace_size(int64_t batch, int64_t seq_len,
+                                                             int64_t num_heads, int64_t head_size,
+                                                             int64_t total_kv) {
+    // As many splits as the call would use: whole CUs over the tiles these rows fill, of
+    // at least 512 keys each.
+    const int64_t rows = std::max<int64_t>(1, batch * seq_len * num_heads);
+    const int64_t splits = std::min<int64_t>({(int64_t)kMaxPrefillSplits, 256 * kAttnRows / rows,
+                                              (std::max<int64_t>(total_kv, 0) + 511) / 512});
+    return gqa_workspace(batch, seq_len, num_heads, head_size, total_kv,
+                         std::max<int64_t>(splits, kPrefillSplits));
 }
 
 // Launch of the one-token decode kernel for G query heads per KV head. When the
@@ -2069,7 +1910,7 @@ static int run_gqa(const void* query, const void* key, const void* value, const 
     const int G = H / KV;
     const float sc = scale != 0.f ? scale : 1.0f / sqrtf((float)hd);
 
-    size_t need = ortmi_group_query_attention_workspace_size(B, S, H, hd, nkeys);
+    size_t need = gqa_workspace(B, S, H, hd, nkeys, kPrefillSplits);
     if (!ws || ws_bytes < need)
         return fail(ORTMI_E_WORKSPACE, "GroupQueryAttention: workspace too small");
     T* qrot = static_cast<T*>(ws);
@@ -2117,41 +1958,52 @@ static int run_gqa(const void* query, const void* key, const void* value, const 
                            (int64_t)H * hd, (const int*)nullptr);
         return check_launch("gqa_merge");
     }
-    hipLaunchKernelGGL((gqa_prep_kernel<T>), dim3(B * S, (H + KV + kPrepHeads - 1) / kPrepHeads),
-                       dim3(64 * kPrepHeads), kPrepHeads * hd * sizeof(float), st,
-                       q, k, v, static_cast<const T*>(cos_c), static_cast<const T*>(sin_c), half,
-                       interleaved, qrot, static_cast<T*>(pk), static_cast<T*>(pv), B, S, H, KV,
-                       hd, pcap, vp, q_stride, kv_stride);
+    // Rotary dims that fill the head, on 16-byte pieces, are rotated by the tile kernel as
+    // it loads the queries; otherwise the prep kernel stages rotated queries.
+    const bool pieces = (!cos_c || 2 * half == hd) && a16(q) && a16(k) && a16(v) && a16(cos_c) &&
+                        a16(sin_c);
+    QueryRows<T> rows{qrot, (int64_t)H * hd, nullptr, nullptr, interleaved};
+    if (pieces) {
+        rows = {q, q_stride, static_cast<const T*>(cos_c), static_cast<const T*>(sin_c),
+                interleaved};
+        const int64_t items = (int64_t)B * S * KV * (hd / 16);
+        hipLaunchKernelGGL((gqa_kv_rows_kernel<T>), dim3((unsigned)((items + 255) / 256)),
+                           dim3(256), 0, st, k, v, rows.cos, rows.sin, interleaved,
+                           static_cast<T*>(pk), static_cast<T*>(pv), S, KV, hd, pcap, vp,
+                           kv_stride, items);
+    } else {
+        hipLaunchKernelGGL((gqa_prep_kernel<T>),
+                           dim3(B * S, (H + KV + kPrepHeads - 1) / kPrepHeads),
+                           dim3(64 * kPrepHeads), kPrepHeads * hd * sizeof(float), st, q, k, v,
+                           static_cast<const T*>(cos_c), static_cast<const T*>(sin_c), half,
+                           interleaved, qrot, static_cast<T*>(pk), static_cast<T*>(pv), B, S, H,
+                           KV, hd, pcap, vp, q_stride, kv_stride);
+    }
     if (int rc = check_launch("gqa_prep")) return rc;
-    const int QT = std::max(1, tile_rows_for<T>(HD, kGqaTileWaves) / G);
-    const int tiles = (S + QT - 1) / QT;
-    DenseKV dk{pk, pv, pcap, KV};
-    // Key splits when the tiles alone leave CUs idle (a 512-token decoder prefill
-    // has 50 tiles): about two workgroups per CU, chunks of at least 128 keys, at
-    // most kPrefillSplits; the splits are merged per (token, head) row.
+    // Key splits when the tiles alone leave CUs idle: one workgroup per CU (its LDS and
+    // registers fill one), chunks of at least 512 keys (4 steps), as many as the
+    // workspace has room for; the splits are merged per (token, head) row.
     int chunk = nkeys, ns = 1;
+    const int64_t prows = (int64_t)B * S * H;
+    const size_t qbytes = align_up((size_t)prows * hd * 4);
     {
-        const int64_t wgs = (int64_t)B * tiles * KV;
-        const int64_t want = std::min<int64_t>(
-            kPrefillSplits, (2LL * device_cu_count() + wgs - 1) / std::max<int64_t>(wgs, 1));
+        const int QT = std::max(1, kAttnRows / G);
+        const int64_t wgs = (int64_t)B * ((S + QT - 1) / QT) * KV;
+        const size_t per_split = (size_t)prows * (hd + 2) * 4;
+        const int64_t room = (int64_t)((ws_bytes - qbytes - align_up((size_t)prows * 4)) / per_split);
+        const int64_t want =
+            std::min<int64_t>({(int64_t)kMaxPrefillSplits, room, device_cu_count() / wgs});
         if (want > 1) {
-            chunk = (int)std::max<int64_t>(128, ((nkeys + want - 1) / want + 63) / 64 * 64);
+            chunk = (int)std::max<int64_t>(512, ((nkeys + want - 1) / want + 63) / 64 * 64);
             ns = (nkeys + chunk - 1) / chunk;
         }
     }
-    float* ppart = nullptr;
-    int* prow = nullptr;
-    if (ns > 1) {
-        char* base = static_cast<char*>(ws) + align_up((size_t)B * S * H * hd * 4);
-        ppart = reinterpret_cast<float*>(base);
-        prow = reinterpret_cast<int*>(base + align_up((size_t)B * S * H * kPrefillSplits *
-                                                      (hd + 2) * 4));
-    }
-    hipLaunchKernelGGL((gqa_tile_kernel<T, HD>), dim3(B * tiles, KV, ns),
-                       dim3(tile_threads<T, HD, kGqaTileWaves>()), 0, st, qrot,
-                       dk, S, QT, tiles, G, H, vp, sc, static_cast<T*>(output), chunk, ns, ppart,
-                       prow);
-    if (int rc = check_launch("gqa_tile")) return rc;
+    int* prow = reinterpret_cast<int*>(static_cast<char*>(ws) + qbytes);
+    float* ppart = reinterpret_cast<float*>(static_cast<char*>(ws) + qbytes +
+                                            align_up((size_t)prows * 4));
+    if (int rc = gqa_tile<T>(rows, static_cast<const T*>(pk), static_cast<const T*>(pv), pcap, B, S,
+                             H, KV, hd, vp, sc, static_cast<T*>(output), chunk, ns, ppart, prow, st))
+        return rc;
     if (ns == 1) return ORTMI_OK;
     hipLaunchKernelGGL((paged_merge_kernel<T>), dim3((unsigned)(B * S), (unsigned)H), dim3(128), 0,
                        st, ppart, static_cast<T*>(output), ns, prow, hd, H, (const float*)nullptr);
@@ -2200,21 +2052,24 @@ extern "C" int ortmi_group_query_attention(
     if (shared_c)
         ORTMI_REQUIRE(total_sequence_length <= past_cap,
                       "GroupQueryAttention: total_sequence_length exceeds the KV buffer capacity");
-    // Head 96 runs the one-token decode on the fast kernel (16-lane groups with 4
-    // padding lanes); prompts, and decode steps the fast kernel does not take
-    // (unaligned tensors, more than 8 query heads per KV head, a rotary half that is
-    // not a multiple of 8), go to the generic kernels.
-    if (head_size == 96) {
+    // The generic kernels take what the matrix-core tiles do not: present tensors that are
+    // not 16-byte aligned, and head 96's decode steps that the fast kernel does not take
+    // (unaligned tensors, more than 8 query heads per KV head, a rotary half that is not a
+    // multiple of 8).
+    if (dtype == ORTMI_F16 || dtype == ORTMI_BF16) {
         const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
         const bool packed = key == nullptr;
-        const void* kk = packed ? static_cast<const char*>(query) + num_heads * 96 * 2 : key;
-        const void* vv = packed ? static_cast<const char*>(query) + (num_heads + kv_num_heads) * 96 * 2
+        const int64_t hb = head_size * 2;
+        const void* kk = packed ? static_cast<const char*>(query) + num_heads * hb : key;
+        const void* vv = packed ? static_cast<const char*>(query) + (num_heads + kv_num_heads) * hb
                                 : value;
-        const bool fast = seq_len == 1 && num_heads / kv_num_heads <= 8 && dtype != ORTMI_F32 &&
+        const bool fast = num_heads / kv_num_heads <= 8 &&
                           (!rotary || rotary_interleaved || rotary_half % 8 == 0) && a16(query) &&
                           a16(kk) && a16(vv) && a16(present_key) && a16(present_value) &&
                           (past_cap == 0 || (a16(past_key) && a16(past_value)));
-        if (!fast)
+        const bool tiles = a16(present_key) && a16(present_value);
+        const bool decode = seq_len == 1 && (fast || head_size == 96);
+        if (decode ? !fast : !tiles)
             return ortmi_group_query_attention_ex(
                 query, key, value, past_key, past_value, past_cap, total_sequence_length,
                 cos_cache, sin_cache, rotary_half, max_pos, nullptr, nullptr, 1e-6f, nullptr, 0, 0,
@@ -2422,7 +2277,7 @@ extern "C" int ortmi_group_query_attention_noalloc(
     int64_t vp = (int64_t)total_sequence_length - seq_len;
     if (vp < 0 || vp > past_cap) vp = past_cap;
     const size_t need =
-        ortmi_group_query_attention_workspace_size(batch, seq_len, num_heads, head_size, vp + seq_len);
+        gqa_workspace(batch, seq_len, num_heads, head_size, vp + seq_len, kPrefillSplits);
     if (need > kGqaScratchBytes)
         return fail(ORTMI_E_WORKSPACE,
                     "GroupQueryAttention (no-alloc): needs " + std::to_string(need) +
@@ -2442,7 +2297,9 @@ extern "C" int ortmi_group_query_attention_noalloc(
 static int paged_max_tiles(int64_t T, int64_t batch, int QT) {
     return (int)((T + QT - 1) / QT + batch);
 }
-static int paged_qt(int G) { return std::max(1, kTileRows / G); }
+// Tokens per tile that the workspace's tile map is sized for: fewer than the tile kernel
+// takes, so that the map bounds its layout too.
+static int paged_qt(int G) { return std::max(1, 64 / G); }
 // Keys per split: at least 512, and at most 8 splits per row (bounds the partials).
 static int paged_nsplit(int64_t max_context, int& chunk) {
     const int64_t c = std::max<int64_t>(512, ((max_context + 7) / 8 + 63) / 64 * 64);
@@ -2645,7 +2502,7 @@ static int run_paged(const void* query, const void* key, const void* value, void
     const int G = H / KV;
     // Tiles of the kernel used for T (the workspace is sized for the smaller tile,
     // which gives more tiles, so it bounds this layout too).
-    const int QT = std::max(1, tile_rows_for<T>(VHD, kPagedTileWaves) / G);
+    const int QT = std::max(1, 32 * kPagedTileWaves / G);
     const int mt = paged_max_tiles(T_, batch, QT);
     int chunk;
     const int ns = paged_nsplit(max_context, chunk);
@@ -2721,7 +2578,7 @@ static int run_paged(const void* query, const void* key, const void* value, void
     }
     const unsigned tile_wgs = (unsigned)(kXcds * (int64_t)mt * ((KV * ns + kXcds - 1) / kXcds));
     hipLaunchKernelGGL((paged_tile_kernel<T, HD, VHD>), dim3(tile_wgs),
-                       dim3(tile_threads<T, VHD, kPagedTileWaves>()), 0, st, tiles,
+                       dim3(64 * kPagedTileWaves), 0, st, tiles,
                        count, cum, past, pk, qrot, G, H, sc, sink ? sink32 : nullptr, chunk, ns,
                        static_cast<T*>(output), part, nsplit_row, dec ? 1 : 0, mt);
     if (int rc = check_launch("paged_tile")) return rc;

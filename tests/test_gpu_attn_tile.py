@@ -1,0 +1,127 @@
+"""GPU parity of the GroupQueryAttention prompt tiles against 64-bit attention, at the edges
+of the tile (128 query rows, key blocks of 64 shared by two groups of waves) and of its
+dispatch (key splits, rotary in the tile or staged, tensors that are not aligned).
+
+Bound: rotated queries and keys are rounded to the type on both sides (a rounding that falls
+the other way moves a score by one unit of one product, a few 2^-p of it), the probabilities
+are rounded once (head 96: not), and so is the output: u * (4 P|V| + |out|) with u the
+type's unit roundoff, P the exact probabilities."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+U = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
+DT = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+
+
+def rope(x, cos, sin, pos0, interleaved, dt):
+    """x [B, S, heads, hd] float64, rotated and rounded to dt."""
+    half = cos.shape[1]
+    c = cos[pos0:pos0 + x.shape[1]].double()[None, :, None]
+    s = sin[pos0:pos0 + x.shape[1]].double()[None, :, None]
+    y = x.clone()
+    a, b = (slice(0, 2 * half, 2), slice(1, 2 * half, 2)) if interleaved else \
+        (slice(0, half), slice(half, 2 * half))
+    y[..., a] = x[..., a] * c - x[..., b] * s
+    y[..., b] = x[..., b] * c + x[..., a] * s
+    return y.to(dt).double()
+
+
+def check(ortmi, dt, B, S, past, H, KV, hd, half=None, interleaved=False, shared=True, shift=0,
+          scale=0.0, packed=False):
+    tdt = DT[dt]
+    g = torch.Generator().manual_seed(S * 131 + past + H + hd)
+    half = hd // 2 if half is None else half
+
+    def rnd(*shape):
+        return torch.randn(shape, generator=g).to(tdt)
+
+    def put(t):  # on the GPU, `shift` elements off an aligned address
+        buf = torch.zeros(t.numel() + shift, dtype=tdt, device="cuda")
+        buf[shift:] = t.flatten().cuda()
+        return buf[shift:].view(t.shape)
+
+    q, k, v = rnd(B, S, H * hd), rnd(B, S, KV * hd), rnd(B, S, KV * hd)
+    cap = past + S + (5 if shared else 0)
+    pk, pv = rnd(B, KV, cap if shared else past, hd), rnd(B, KV, cap if shared else past, hd)
+    ang = torch.rand((past + S, max(half, 1)), generator=g) * 6
+    cos, sin = ang.cos().to(tdt), ang.sin().to(tdt)
+    kw = dict(num_heads=H, kv_num_heads=KV, scale=scale, rotary_interleaved=int(interleaved),
+              do_rotary=int(half > 0))
+    dpk, dpv = put(pk), put(pv)
+    if shared:
+        kw.update(present_key=dpk, present_value=dpv)
+    qkv = (put(torch.cat([q, k, v], -1)), None, None) if packed else (put(q), put(k), put(v))
+    out, ok, ov = ortmi.group_query_attention(*qkv, dpk, dpv, None, past + S,
+                                              cos.cuda() if half else None,
+                                              sin.cuda() if half else None, **kw)
+    qd, kd = q.double().reshape(B, S, H, hd), k.double().reshape(B, S, KV, hd)
+    if half:
+        qd, kd = (rope(x, cos, sin, past, interleaved, tdt) for x in (qd, kd))
+    keys = torch.cat([pk[:, :, :past].double(), kd.transpose(1, 2)], 2)
+    vals = torch.cat([pv[:, :, :past].double(), v.double().reshape(B, S, KV, hd).transpose(1, 2)], 2)
+    rep = torch.arange(H) // (H // KV)
+    sc = qd.transpose(1, 2) @ keys[:, rep].transpose(-1, -2) * (scale or 1 / math.sqrt(hd))
+    hide = torch.arange(past + S)[None] > past + torch.arange(S)[:, None]
+    p = torch.softmax(sc.masked_fill(hide, -math.inf), -1)
+    want = (p @ vals[:, rep]).transpose(1, 2)
+    mag = (p @ vals[:, rep].abs()).transpose(1, 2)
+    got = out.double().cpu().reshape(B, S, H, hd)
+    if dt == "f32":
+        bound = 2.0 ** -24 * ((past + S + 8 * hd) * mag + want.abs())
+    else:
+        bound = U[dt] * (4 * mag + want.abs())
+    excess = ((got - want).abs() - bound).max().item()
+    assert excess <= 1e-6, f"max excess {excess:.3e}"
+    n = past + S
+    err = (ok.double().cpu()[:, :, :n] - keys).abs().max().item()
+    assert err <= (2.0 ** -20 if dt == "f32" else 2 * U[dt]) * keys.abs().max().item()
+    assert torch.equal(ov.double().cpu()[:, :, :n], vals)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("hd", [64, 96, 128])
+@pytest.mark.parametrize("B,S,past,H,KV", [
+    (1, 2, 0, 4, 4),       # one block, the second key group without work
+    (2, 33, 31, 14, 2),    # 18 tokens of 7 heads to a tile, a block cut at 64
+    (1, 65, 0, 8, 8),      # one head per tile row group, one key past a block
+    (1, 128, 64, 4, 1),
+    (3, 129, 62, 16, 4),   # a tile with one token; odd number of blocks
+    (1, 5, 1500, 32, 8),   # few rows, many keys: splits, merged
+    (1, 20, 2000, 24, 8),  # the last split shorter
+])
+def test_gqa_tile(ortmi, dt, hd, B, S, past, H, KV):
+    check(ortmi, dt, B, S, past, H, KV, hd)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("opt", [
+    dict(interleaved=True), dict(half=0), dict(half=16), dict(half=24, interleaved=True),
+    dict(shared=False), dict(shift=1), dict(shift=3, interleaved=True), dict(scale=-0.2),
+    dict(packed=True)])
+@pytest.mark.parametrize("hd", [64, 96, 128])
+def test_gqa_tile_options(ortmi, dt, hd, opt):
+    check(ortmi, dt, 2, 37, 70, 8, 2, hd, **opt)
+
+
+def test_gqa_tile_head96_keeps_probabilities(ortmi):
+    """Head 96 rounds no probability: with large values that cancel, the error stays at that
+    of fp32 arithmetic and one rounding of the output."""
+    B, S, H, hd = 1, 64, 2, 96
+    g = torch.Generator().manual_seed(3)
+    q, k = (torch.randn((B, S, H * hd), generator=g).half() * 0.1 for _ in range(2))
+    v = (torch.randn((B, S, H * hd), generator=g).sign() * 1000).half()
+    z = torch.zeros((B, H, 0, hd), dtype=torch.float16, device="cuda")
+    out, _, _ = ortmi.group_query_attention(q.cuda(), k.cuda(), v.cuda(), z, z, None, S, None, None,
+                                            num_heads=H, kv_num_heads=H)
+    qd, kd, vd = (x.double().reshape(S, H, hd).transpose(0, 1) for x in (q, k, v))
+    sc = (qd @ kd.transpose(-1, -2)) / math.sqrt(hd)
+    sc = sc.masked_fill(torch.ones(S, S).triu(1).bool(), -math.inf)
+    want = (torch.softmax(sc, -1) @ vd).transpose(0, 1).reshape(S, H * hd)
+    err = (out.double().cpu()[0] - want).abs()
+    assert (err <= 2.0 ** -11 * want.abs() + 1000 * 2.0 ** -19).all(), err.max().item()
