@@ -1720,73 +1720,48 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
 
 // Merge of split rows, one workgroup per (token, head) row, with the optional
 // head sink folded in. Rows with a split count of 0 were written directly.
+// One wave per row, two dims per lane: lane i weighs split i, and all of a row's loads go
+// out together. Bound by the partials' bytes: 1052 tokens of 32 heads of 128, 4 splits on
+// average, 31 us with a workgroup of two waves per row and one dim per thread.
+constexpr int kMergeRows = 4;  // waves per workgroup
 template <typename T>
-__global__ __launch_bounds__(128) void paged_merge_kernel(const float* __restrict__ part,
-                                                          T* __restrict__ out, int nsplit,
-                                                          const int* __restrict__ nsplit_row,
-                                                          int vhd, int H,
-                                                          const float* __restrict__ sink) {
-    const int64_t tok = blockIdx.x;
-    const int h = blockIdx.y;
-    const int64_t r = tok * H + h;
-    const int ns = min(nsplit, nsplit_row[r]);
+__global__ __launch_bounds__(64 * kMergeRows) void paged_merge_kernel(
+    const float* __restrict__ part, T* __restrict__ out, int nsplit,
+    const int* __restrict__ nsplit_row, int vhd, int H, const float* __restrict__ sink,
+    int64_t rows) {
+    const int lane = threadIdx.x & 63;
+    const int64_t r = (int64_t)blockIdx.x * kMergeRows + (threadIdx.x >> 6);
+    if (r >= rows) return;
+    const int ns = min(nsplit, nsplit_row[r]);  // at most 64 (the callers' split rules)
     if (ns <= 0) return;
     const float* p = part + r * nsplit * (vhd + 2);
-    if (ns <= kMergeFast && vhd <= 128) {
-        // Every value a thread needs in one batch of loads (splits past the count
-        // read zeros without an access), merged in registers.
-        const uint32_t bytes = (uint32_t)(ns * (vhd + 2)) * 4u;
-        const __amdgpu_buffer_rsrc_t rp = buffer_rsrc(p, bytes);
-        const int d = min((int)threadIdx.x, vhd - 1);
-        float mv[kMergeFast], lv[kMergeFast], ov[kMergeFast];
-#pragma unroll
-        for (int i = 0; i < kMergeFast; ++i) {
-            const uint32_t row = (uint32_t)(i * (vhd + 2)) * 4u;
-            const bool in = i < ns;
-            mv[i] = __uint_as_float(
-                __builtin_amdgcn_raw_buffer_load_b32(rp, in ? row + vhd * 4u : bytes, 0, 0));
-            lv[i] = __uint_as_float(
-                __builtin_amdgcn_raw_buffer_load_b32(rp, in ? row + vhd * 4u + 4u : bytes, 0, 0));
-            ov[i] = __uint_as_float(
-                __builtin_amdgcn_raw_buffer_load_b32(rp, in ? row + d * 4u : bytes, 0, 0));
-        }
-        float M = sink ? sink[h] : -INFINITY;
-#pragma unroll
-        for (int i = 0; i < kMergeFast; ++i)
-            if (i < ns) M = fmaxf(M, mv[i]);
-        float L = sink && M != -INFINITY ? __expf(sink[h] - M) : 0.f, acc = 0.f;
-#pragma unroll
-        for (int i = 0; i < kMergeFast; ++i) {
-            const float w = i < ns && mv[i] != -INFINITY ? __expf(mv[i] - M) : 0.f;
-            L = fmaf(w, lv[i], L);
-            acc = fmaf(w, ov[i], acc);
-        }
-        if ((int)threadIdx.x < vhd)
-            out[tok * ((int64_t)H * vhd) + (int64_t)h * vhd + threadIdx.x] =
-                from_f32<T>(L > 0.f ? acc / L : 0.f);
-        return;
-    }
-    float M = -INFINITY;
-    for (int i = 0; i < ns; ++i) M = fmaxf(M, p[i * (vhd + 2) + vhd]);
-    if (sink) M = fmaxf(M, sink[h]);
-    float L = 0.f;
-    for (int i = 0; i < ns; ++i) {
-        const float m = p[i * (vhd + 2) + vhd];
-        if (m != -INFINITY) L += p[i * (vhd + 2) + vhd + 1] * __expf(m - M);
-    }
-    if (sink) L += __expf(sink[h] - M);
+    const bool mine = lane < ns;
+    const float m = mine ? p[lane * (vhd + 2) + vhd] : -INFINITY;
+    const float lp = mine ? p[lane * (vhd + 2) + vhd + 1] : 0.f;
+    const float sk = sink ? sink[r % H] : -INFINITY;
+    const float M = fmaxf(wave_max(m), sk);
+    const float w = m != -INFINITY ? __expf(m - M) : 0.f;
+    const float L = wave_sum(w * lp) + (sk != -INFINITY ? __expf(sk - M) : 0.f);
     const float inv = L > 0.f ? 1.0f / L : 0.f;
-    T* o = out + tok * ((int64_t)H * vhd) + (int64_t)h * vhd;
-    for (int d = threadIdx.x; d < vhd; d += blockDim.x) {
-        float acc = 0.f;
-        for (int i = 0; i < ns; ++i) {
-            const float m = p[i * (vhd + 2) + vhd];
-            if (m != -INFINITY) acc += p[i * (vhd + 2) + d] * __expf(m - M);
+    for (int d = 2 * lane; d < vhd; d += 128) {
+        float a = 0.f, b = 0.f;
+        for (int i0 = 0; i0 < ns; i0 += 8) {
+            float2 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                v[i] = *reinterpret_cast<const float2*>(p + min(i0 + i, ns - 1) * (vhd + 2) + d);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float wi = __shfl(w, i0 + i, 64);  // 0 past the last split
+                a = wi != 0.f ? fmaf(v[i].x, wi, a) : a;
+                b = wi != 0.f ? fmaf(v[i].y, wi, b) : b;
+            }
         }
-        o[d] = from_f32<T>(acc * inv);
+        T* o = out + r * vhd + d;
+        o[0] = from_f32<T>(a * inv);
+        o[1] = from_f32<T>(b * inv);
     }
 }
-
 
 __global__ void sink_to_f32_kernel(const void* src, int dtype, float* dst, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2084,8 +2059,9 @@ static int run_gqa(const void* query, const void* key, const void* value, const 
                              H, KV, hd, vp, sc, static_cast<T*>(output), chunk, ns, ppart, prow, st))
         return rc;
     if (ns == 1) return ORTMI_OK;
-    hipLaunchKernelGGL((paged_merge_kernel<T>), dim3((unsigned)(B * S), (unsigned)H), dim3(128), 0,
-                       st, ppart, static_cast<T*>(output), ns, prow, hd, H, (const float*)nullptr);
+    hipLaunchKernelGGL((paged_merge_kernel<T>), dim3((unsigned)((prows + kMergeRows - 1) / kMergeRows)),
+                       dim3(64 * kMergeRows), 0, st, ppart, static_cast<T*>(output), ns, prow, hd,
+                       H, (const float*)nullptr, prows);
     return check_launch("gqa_tile_merge");
 }
 
@@ -2676,9 +2652,10 @@ static int run_paged(const void* query, const void* key, const void* value, void
                        static_cast<T*>(output), part, nsplit_row, dec ? 1 : 0, mt);
     if (int rc = check_launch("paged_tile")) return rc;
     if (ns > 1) {
-        hipLaunchKernelGGL((paged_merge_kernel<T>), dim3((unsigned)T_, (unsigned)H), dim3(128), 0, st, part,
-                           static_cast<T*>(output), ns, nsplit_row, VHD, H,
-                           sink ? sink32 : nullptr);
+        hipLaunchKernelGGL((paged_merge_kernel<T>),
+                           dim3((unsigned)((prow + kMergeRows - 1) / kMergeRows)),
+                           dim3(64 * kMergeRows), 0, st, part, static_cast<T*>(output), ns,
+                           nsplit_row, VHD, H, sink ? sink32 : nullptr, prow);
         return check_launch("paged_merge");
     }
     return ORTMI_OK;
