@@ -2,7 +2,7 @@
 // fp32 tensors, per-head QK RMS-norm (inputs 14/15), an additive attention_bias
 // (input 10) and head sizes other than 64/128 (multiples of 16 up to 256).
 //
-// Two kernels:
+// Three kernels:
 //  - gqa_ex_prep_kernel: one wave per (token, head) vector. Q heads: optional
 //    RMS-norm, optional RoPE at position valid_past + s, each step rounded to the
 //    op dtype as the reference materialises it (rust/src/ops/attention.rs:663-708),
@@ -12,6 +12,8 @@
 //    head). Team t scores keys t, t+16, ... (a 16-lane dot product reduced inside a
 //    DPP row), adds the bias, and keeps an online softmax; the 16 team states are
 //    merged through LDS. Causal: query s attends keys [0, valid_past + s].
+//  - gqa_f32_tile_kernel: fp32 at head sizes 64, 96 and 128 without a bias, on the fp32
+//    matrix cores.
 // The KV contract (shared buffer vs growing, attention.rs:636-651) is that of
 // ortmi_group_query_attention.
 //
@@ -345,6 +347,199 @@ __global__ __launch_bounds__(256) void gqa_ex_attn_kernel(
     }
 }
 
+// fp32 without bias on the fp32 matrix cores (v_mfma_f32_32x32x2_f32: every product and sum
+// in fp32, as in the kernel above). A workgroup takes 32 query rows (token, head of the
+// group) of one KV head, and its 8 waves take every eighth tile of 32 keys, straight from
+// memory: the rows of a tile are read once per workgroup, and the waves' states are merged
+// through LDS at the end.
+//   S^T = K Q^T    lane l: key (query) l & 31, step s: dims s and HD/2 + s for the lane
+//                  halves, so a lane's share of a row is contiguous
+//   O^T += V^T P^T step e: the lane halves' keys of accumulator e, P straight from the
+//                  softmax's registers
+// Bound: short prompts by the latency of a tile (two per wave at 512 keys), long ones by
+// the fp32 matrix rate (64 cycles per instruction of 4096 operations). One workgroup per
+// query row before: 512 tokens, 14 heads of 64 on 2: 114 -> 26 us; B 2, 300 tokens behind 2000,
+// 32 heads of 128 on 8: 4400 -> 594 us; B 2, one token behind 2048: 445 -> 166 us. Errors
+// against 64 bits 1.4e-7 -> 1.3e-7, 2.8e-7 -> 1.9e-7, 2.8e-7 -> 1.9e-7.
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+constexpr int kF32Rows = 32, kF32Keys = 32, kF32Waves = 8;
+// S^T over pieces [I, I + N) of the head dims.
+template <int I, int N>
+__device__ __forceinline__ f32x16_t f32_dot_tree(const float4* k4, const float4* q4) {
+    if constexpr (N == 1) {
+        f32x16_t a;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) a[e] = 0.f;
+        a = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[I].x, q4[I].x, a, 0, 0, 0);
+        a = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[I].y, q4[I].y, a, 0, 0, 0);
+        a = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[I].z, q4[I].z, a, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_32x32x2f32(k4[I].w, q4[I].w, a, 0, 0, 0);
+    } else {
+        const f32x16_t a = f32_dot_tree<I, N / 2>(k4, q4);
+        const f32x16_t b = f32_dot_tree<I + N / 2, N - N / 2>(k4, q4);
+        return a + b;
+    }
+}
+template <int HD>
+__global__ __launch_bounds__(64 * kF32Waves, 1) void gqa_f32_tile_kernel(
+    const float* __restrict__ qf, const float* __restrict__ pk, const float* __restrict__ pv,
+    float* __restrict__ out, int S, int H, int KV, int64_t pcap, int vp, float scale, int tiles) {
+    constexpr int DT = HD / 32, HALF = HD / 2;
+    __shared__ float s_o[kF32Waves][DT * 16 * 64];
+    __shared__ float s_m[kF32Waves][32], s_l[kF32Waves][32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 31, hh = lane >> 5;
+    const int G = H / KV, rows = S * G;
+    // Tiles of later tokens, which walk more keys, first.
+    const int tile = tiles - 1 - (int)blockIdx.x % tiles, bkv = (int)blockIdx.x / tiles;
+    const int b = bkv / KV, kvh = bkv % KV;
+    const int r0 = tile * kF32Rows, r = min(r0 + li, rows - 1);
+    const int tok = r / G, head = kvh * G + r % G;
+    const int nk = vp + min(r0 + kF32Rows - 1, rows - 1) / G + 1;  // causal bound of the tile
+    const int seen_all = vp + r0 / G;  // keys up to here are visible to every row
+    const int last = vp + tok;         // this row's last key
+    const float* const kbase = pk + (int64_t)bkv * pcap * HD;
+    const float* const vbase = pv + (int64_t)bkv * pcap * HD;
+
+    float4 q4[HALF / 4];
+    {
+        const float* qrow = qf + (((int64_t)b * S + tok) * H + head) * HD + hh * HALF;
+#pragma unroll
+        for (int i = 0; i < HALF / 4; ++i) {
+            q4[i] = *reinterpret_cast<const float4*>(qrow + 4 * i);
+            if (scale < 0.f) q4[i] = make_float4(-q4[i].x, -q4[i].y, -q4[i].z, -q4[i].w);
+        }
+    }
+    constexpr float kLog2e = 1.4426950408889634f;
+    // Maxima are kept of the raw scores (a negative scale turns the sign of Q) and P is
+    // exp2((s - m) * sc2): the difference is exact or nearly so where P is large, so that
+    // no rounding of a large product reaches the exponent.
+    const float sc2 = fabsf(scale) * kLog2e;
+    float m = -INFINITY, l = 0.f;
+    f32x16_t o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[d][e] = 0.f;
+
+    for (int kb = wave * kF32Keys; kb < nk; kb += kF32Waves * kF32Keys) {
+        // Rows past the end read the last one; their keys are masked.
+        const float* krow = kbase + (int64_t)min(kb + li, nk - 1) * HD + hh * HALF;
+        float4 k4[HALF / 4];
+#pragma unroll
+        for (int i = 0; i < HALF / 4; ++i) k4[i] = *reinterpret_cast<const float4*>(krow + 4 * i);
+        // The sum over the head dims as a tree over pieces of four steps: summed in one chain
+        // the error was twice that of the kernel above (B 2, one token, 2048 keys, head 128:
+        // 5.0e-7 relative to 64 bits against 2.8e-7).
+        f32x16_t st = f32_dot_tree<0, HALF / 4>(k4, q4);
+        // Accumulator e holds key 8 (e / 4) + 4 hh + e % 4 of query li.
+        const bool part = kb + kF32Keys - 1 > seen_all;
+        float mt = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int j = kb + 8 * (e / 4) + 4 * hh + (e & 3);
+            st[e] = !part || j <= last ? st[e] : -INFINITY;
+            mt = fmaxf(mt, st[e]);
+        }
+        const LanePair pm = swap32(mt);
+        const float mn = fmaxf(m, fmaxf(pm.a, pm.b));
+        const float corr = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * sc2);
+        const float ref = mn == -INFINITY ? 0.f : mn;
+        float lt = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            st[e] = __builtin_amdgcn_exp2f((st[e] - ref) * sc2);
+            lt += st[e];
+        }
+        l = l * corr + lt;  // this lane's 16 of the tile's keys
+        m = mn;
+        const float* vcol = vbase + li;
+        auto vrow = [&](int e) {
+            return vcol + (int64_t)min(kb + 8 * (e / 4) + 4 * hh + (e & 3), nk - 1) * HD;
+        };
+        // A hidden key must not reach a row through 0 * infinity: where some keys are hidden
+        // and some values are not finite, the products are taken one key at a time.
+        bool odd = false;
+        if (part) {
+            float z = 0.f;
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+#pragma unroll
+                for (int d = 0; d < DT; ++d) z = fmaf(vrow(e)[d * 32], 0.f, z);
+            odd = __any(z != 0.f);  // NaN
+        }
+        if (!odd) {
+            // Each tile sums on its own, in two chains, before it joins O.
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                f32x16_t t0, t1;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) t0[e] = t1[e] = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    t0 = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow(e)[d * 32], st[e], t0, 0, 0, 0);
+                    t1 = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow(e + 8)[d * 32], st[e + 8], t1, 0,
+                                                              0, 0);
+                }
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o[d][e] = fmaf(o[d][e], corr, t0[e] + t1[e]);
+            }
+        } else {
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o[d][e] *= corr;
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                for (int h2 = 0; h2 < 2; ++h2) {
+                    const int j = kb + 8 * (e / 4) + 4 * h2 + (e & 3);
+                    const float pj = __shfl(st[e], li + 32 * h2, 64);
+                    const float* vr = vbase + (int64_t)min(j, nk - 1) * HD;
+                    if (j > last) continue;
+#pragma unroll
+                    for (int d = 0; d < DT; ++d)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i)
+                            o[d][i] = fmaf(pj, vr[d * 32 + 8 * (i / 4) + 4 * hh + (i & 3)], o[d][i]);
+                }
+        }
+    }
+    const LanePair pl = swap32(l);
+    l = pl.a + pl.b;
+    if (hh == 0) {
+        s_m[wave][li] = m;
+        s_l[wave][li] = l;
+    }
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s_o[wave][(d * 16 + e) * 64 + lane] = o[d][e];
+    __syncthreads();
+    // Four consecutive dims of one row per thread and turn.
+    for (int i = threadIdx.x; i < DT * 4 * 64; i += 64 * kF32Waves) {
+        const int ln = i & 63, q = ln & 31, d = i / 256, e4 = (i >> 6) & 3;
+        if (r0 + q >= rows) continue;
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kF32Waves; ++w) M = fmaxf(M, s_m[w][q]);
+        float den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < kF32Waves; ++w) {
+            // A wave without a visible key has zeros, or NaN from NaN scores.
+            const float f =
+                s_m[w][q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((s_m[w][q] - M) * sc2);
+            den = fmaf(f, s_l[w][q], den);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                num[e] = fmaf(f, s_o[w][(d * 16 + 4 * e4 + e) * 64 + ln], num[e]);
+        }
+        const int tq = (r0 + q) / G, hq = kvh * G + (r0 + q) % G;
+        float* dst = out + (((int64_t)b * S + tq) * H + hq) * HD + d * 32 + 8 * e4 + 4 * (ln >> 5);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[e] = num[e] / den;  // every key masked: 0/0
+    }
+}
+
 template <typename T>
 int run_gqa_ex(const void* query, const void* key, const void* value, const void* past_key,
                const void* past_value, int64_t cap, int total, const void* cos_c,
@@ -389,6 +584,24 @@ int run_gqa_ex(const void* query, const void* key, const void* value, const void
                        static_cast<const T*>(kw), eps, qf, static_cast<T*>(pk),
                        static_cast<T*>(pv), S, H, KV, hd, pcap, vp, nullptr, 0);
     if (int rc = check_launch("gqa_ex_prep")) return rc;
+    if constexpr (std::is_same<T, float>::value) {
+        // Row vectors of 16 bytes: ws and present are read so.
+        const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+        const int64_t tiles = ((int64_t)S * (H / KV) + kF32Rows - 1) / kF32Rows;
+        const int64_t grid = (int64_t)B * KV * tiles;
+        if (!bias && a16(ws) && a16(pk) && (hd == 64 || hd == 96 || hd == 128) &&
+            grid <= 0x7fffffffLL) {
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * kF32Waves), 0, st, qf,
+                                   static_cast<const float*>(pk), static_cast<const float*>(pv),
+                                   static_cast<float*>(output), S, H, KV, pcap, vp, sc, (int)tiles);
+                return check_launch("gqa_f32_tile");
+            };
+            if (hd == 64) return launch(gqa_f32_tile_kernel<64>);
+            if (hd == 96) return launch(gqa_f32_tile_kernel<96>);
+            return launch(gqa_f32_tile_kernel<128>);
+        }
+    }
     hipLaunchKernelGGL((gqa_ex_attn_kernel<T>), dim3(B * S * H), dim3(256), 0, st, qf,
                        static_cast<const T*>(pk), static_cast<const T*>(pv),
                        static_cast<const T*>(bias), sb, sh, ss, static_cast<T*>(output), S, H, KV,

@@ -84,7 +84,7 @@ def check(ortmi, dt, B, S, past, H, KV, hd, half=None, interleaved=False, shared
     assert torch.equal(ov.double().cpu()[:, :, :n], vals)
 
 
-@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("hd", [64, 96, 128])
 @pytest.mark.parametrize("B,S,past,H,KV", [
     (1, 2, 0, 4, 4),       # one block, the second key group without work
@@ -94,6 +94,7 @@ def check(ortmi, dt, B, S, past, H, KV, hd, half=None, interleaved=False, shared
     (3, 129, 62, 16, 4),   # a tile with one token; odd number of blocks
     (1, 5, 1500, 32, 8),   # few rows, many keys: splits, merged
     (1, 20, 2000, 24, 8),  # the last split shorter
+    (2, 1, 300, 6, 3),     # (fp32: one token on the tiles too)
 ])
 def test_gqa_tile(ortmi, dt, hd, B, S, past, H, KV):
     check(ortmi, dt, B, S, past, H, KV, hd)
@@ -107,6 +108,21 @@ def test_gqa_tile(ortmi, dt, hd, B, S, past, H, KV):
 @pytest.mark.parametrize("hd", [64, 96, 128])
 def test_gqa_tile_options(ortmi, dt, hd, opt):
     check(ortmi, dt, 2, 37, 70, 8, 2, hd, **opt)
+
+
+def test_gqa_f32_tile_infinite_value_stays_in_its_rows(ortmi):
+    """An infinite value of a key reaches the rows that see the key and no other."""
+    S, H, hd = 45, 2, 64
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn((1, S, H * hd), generator=g) for _ in range(3))
+    v[0, 20, 3] = math.inf
+    z = torch.zeros((1, H, 0, hd), device="cuda")
+    out, _, _ = ortmi.group_query_attention(q.cuda(), k.cuda(), v.cuda(), z, z, None, S, None, None,
+                                            num_heads=H, kv_num_heads=H)
+    out = out.cpu()[0]
+    assert torch.isfinite(out[:20]).all() and (out[20:, 3] == math.inf).all()
+    out[20:, 3] = 0
+    assert torch.isfinite(out).all()
 
 
 def test_gqa_tile_head96_keeps_probabilities(ortmi):
