@@ -15,9 +15,9 @@
 //    s*(sum(a*q) - zp*sum(a)), one byte-convert and one FMA per code. fp16
 //    activations: codes become exact fp16 (q - zp) pairs and v_dot2_f32_f16
 //    takes two codes per instruction.
-//  * the prefill GEMM (mnb_gemm.hip) - M > kBlkRows, fp16 or bf16, bits 4, bs in
-//    {32, 64, 128}: matrix-core tiles over dequantised weights staged in LDS.
-//  * mnb_blk.hip - smaller batches of those, and bits 8 or fp32 activations at any M:
+//  * the prefill GEMM (mnb_gemm.hip) - prompts, fp16 or bf16, bits 4, bs in {32, 64,
+//    128}: matrix-core tiles over dequantised weights staged in LDS.
+//  * mnb_blk.hip - smaller products of those (mnb_takes_blk), and bits 8 or fp32 activations at any M:
 //    matrix cores fed from registers, K split over the waves of a workgroup.
 //  * mnb_generic - every other form (bs 16, unaligned tensors): fp32 dequant to LDS
 //    and a VALU tile product.
@@ -753,7 +753,7 @@ static int run_mnb(const void* A, const uint8_t* B, const void* S, const uint8_t
                            (reinterpret_cast<uintptr_t>(A) % 16) == 0 && K % 8 == 0 &&
                            (size_t)M * K * 2 <= 0xFFFFFF00ull &&
                            (size_t)N * nb * bs / 2 <= 0xFFFFFF00ull;
-    if (!gemm_form || M <= kBlkRows) {
+    if (!gemm_form || mnb_takes_blk(M, N)) {
         const int rc = bits == 4 ? mnb_blk<T, 4>(a, B, s, Z, y, M, N, K, bs, st)
                                  : mnb_blk<T, 8>(a, B, s, Z, y, M, N, K, bs, st);
         if (rc >= 0) return rc;
@@ -918,7 +918,7 @@ extern "C" int ortmi_matmul_nbits_swiglu_pairs(const void* A, const uint8_t* B,
     half_t* y = static_cast<half_t*>(Y);
     hipStream_t st = as_stream(stream);
     const int m = (int)M, n = (int)N, k = (int)K;
-    if (m > 1 && m <= kBlkRows) {  // the rule of ortmi_matmul_nbits: the same sums
+    if (m > 1 && mnb_takes_blk(m, n)) {  // the rule of ortmi_matmul_nbits: the same sums
         const int rc = mnb_blk<half_t, 4, true>(a, B, s, zero_points, y, m, n, k, (int)block_size, st);
         if (rc >= 0) return rc;
     }

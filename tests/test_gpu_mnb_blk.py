@@ -48,6 +48,9 @@ def _run(ortmi, oracle, dt, M, K, N, bits, block, asym, edit=None):
     (1, 11072, 64, 8, 128, False),
     (5, 360, 130, 8, 64, True),
     (130, 712, 4200, 8, 32, True),
+    (65, 1536, 130, 4, 32, True),   # past 64 rows, too few outputs for the prefill GEMM
+    (200, 896, 515, 4, 64, False),
+    (512, 360, 1030, 4, 32, True),
 ])
 def test_mnb_blk(ortmi, oracle, dt, M, K, N, bits, block, asym):
     got, A, W = _run(ortmi, oracle, dt, M, K, N, bits, block, asym)
