@@ -29,18 +29,27 @@ __device__ __forceinline__ uint4 dequant_word_pairs(uint32_t w, half2_t zoff, ha
 }
 
 
-// bf16 weights: (q - zp) is formed exactly in fp16 as above, widened and scaled
-// in fp32, and rounded once to bf16 (bf16((q - zp) * s)).
+// bf16 weights, in the codes' own order (the activations then need no permutation): a byte
+// 0000qqqq read as fp8 (e4m3) is q * 2^-9 exactly, and q * s - zp * s is exact in fp32 (s has
+// 8 mantissa bits), so that only the conversion rounds: bf16((q - zp) * s). 19 vector
+// instructions per 8 codes; by way of fp16 pairs, widened and scaled in fp32, 32 (1999 x
+// 17920 x 1536, block 128: 153 us).
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ uint4 dequant_word_pairs_bf16(uint32_t w, half2_t zoff, float s) {
+__device__ __forceinline__ uint4 dequant_word_bf16(uint32_t w, float s512, float zs) {
+    const uint32_t ev = w & 0x0F0F0F0Fu, od = (w >> 4) & 0x0F0F0F0Fu;
     uint32_t r[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t m = ((w >> (4 * j)) & 0x000F000Fu) | 0x64006400u;
-        const half2_t h = __builtin_bit_cast(half2_t, m) - zoff;
-        const bf16x2_t v = {(__bf16)((float)h.x * s), (__bf16)((float)h.y * s)};
-        r[j] = __builtin_bit_cast(uint32_t, v);
+    for (int h = 0; h < 2; ++h) {
+        const auto e = h ? __builtin_amdgcn_cvt_pk_f32_fp8((int)ev, true)
+                         : __builtin_amdgcn_cvt_pk_f32_fp8((int)ev, false);
+        const auto o = h ? __builtin_amdgcn_cvt_pk_f32_fp8((int)od, true)
+                         : __builtin_amdgcn_cvt_pk_f32_fp8((int)od, false);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const bf16x2_t v = {(__bf16)fmaf(e[i], s512, zs), (__bf16)fmaf(o[i], s512, zs)};
+            r[2 * h + i] = __builtin_bit_cast(uint32_t, v);
+        }
     }
     return make_uint4(r[0], r[1], r[2], r[3]);
 }
@@ -50,28 +59,26 @@ __device__ __forceinline__ uint4 dequant_word_pairs_bf16(uint32_t w, half2_t zof
 // pairs, and the 32x32x16 matrix-core step.
 template <typename T>
 struct GemmDq {
-    half2_t zoff;
-    half2_t s2;  // fp16: the scale as a pair
-    float s;     // bf16: the scale in fp32
+    half2_t zoff, s2;  // fp16: 1024 + zero point and the scale, as pairs
+    float s512, zs;    // bf16: 512 * scale, -zero point * scale
 };
 template <typename T>
 __device__ __forceinline__ GemmDq<T> gemm_dq(float zf, uint16_t sbits) {
-    GemmDq<T> d;
-    d.zoff = half2_t{(half_t)(1024.f + zf), (half_t)(1024.f + zf)};
+    GemmDq<T> d{};
     if constexpr (std::is_same<T, half_t>::value) {
         const half_t sh = __builtin_bit_cast(half_t, sbits);
+        d.zoff = half2_t{(half_t)(1024.f + zf), (half_t)(1024.f + zf)};
         d.s2 = half2_t{sh, sh};
-        d.s = 0.f;
     } else {
-        d.s2 = half2_t{(half_t)0.f, (half_t)0.f};
-        d.s = to_f32(sbits);
+        d.s512 = to_f32(sbits) * 512.f;
+        d.zs = -zf * to_f32(sbits);
     }
     return d;
 }
 template <typename T>
 __device__ __forceinline__ uint4 gemm_dequant(uint32_t w, const GemmDq<T>& d) {
     if constexpr (std::is_same<T, half_t>::value) return dequant_word_pairs(w, d.zoff, d.s2);
-    else return dequant_word_pairs_bf16(w, d.zoff, d.s);
+    else return dequant_word_bf16(w, d.s512, d.zs);
 }
 template <typename T>
 __device__ __forceinline__ float16_t gemm_mfma(half8_t a, half8_t b, float16_t c) {
@@ -218,7 +225,8 @@ __global__ __launch_bounds__(256 * KS) void mnb_gemm4_kernel(const T* __restrict
         for (int p = 0; p < A_VEC; ++p) {
             const int idx = tid + p * 256;
             const int r = idx >> 3, c = (idx & 7) * 8;
-            *reinterpret_cast<uint4*>(&sA[buf][r * kLdsRow + c]) = permute_act8(st.a[p]);
+            *reinterpret_cast<uint4*>(&sA[buf][r * kLdsRow + c]) =
+                std::is_same<T, half_t>::value ? permute_act8(st.a[p]) : st.a[p];
         }
         if constexpr (!BR) {
             const float zf = Z ? (float)nibble(st.z, st.zhi) : 8.f;
