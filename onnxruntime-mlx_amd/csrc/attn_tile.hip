@@ -438,8 +438,10 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
         lsum = pr.a + pr.b;
     }
 
-    // --- the key groups' states, merged by the first --------------------------------
-    {
+    // --- the key groups' states, merged by the first (which alone has a single block) ----
+    if (nblocks <= 1) {
+        if (kg == 1 || !qlive) return;
+    } else {
         constexpr int DK = KC / 8;  // head-dim tiles per K buffer pair (16 KB each)
         static_assert(DT <= 2 * DK, "exchange space");
         float* const x0 = reinterpret_cast<float*>(&sK0[0][0]);
