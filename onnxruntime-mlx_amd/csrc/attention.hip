@@ -166,7 +166,7 @@ __global__ __launch_bounds__(64 * kPrepHeads) void gqa_prep_kernel(
 // loads them: one thread takes the 8 dims from 8c and the 8 from hd/2 + 8c of a (token,
 // KV head), K rotated (rotary dims = hd; cos null: as it is) and V copied to present rows
 // vp + s. Bound by its 16-byte accesses; 2048 tokens of 32 + 8 heads of 128, whose rotated
-// queries went through memory as well: 22 us before.
+// queries went through memory as well: 22 us before, 7.3 us now.
 template <typename T>
 __device__ __forceinline__ void unpack8(u32x4_t w, float (&x)[8]) {
 #pragma unroll
@@ -1367,7 +1367,7 @@ __global__ __launch_bounds__(64 * kPrepHeads) void paged_prep_kernel(
 // The same in 16-byte pieces, without QK norms and with rotary dims that fill the head
 // (or none): one thread takes the 8 dims from 8c and the 8 from hd/2 + 8c of a query or
 // key head of the token; the key heads' threads move the value row too. 1052 tokens of 32
-// + 8 heads of 128: 17.6 us with the kernel above.
+// + 8 heads of 128: 17.6 us with the kernel above, 7.5 us here.
 template <typename T>
 __global__ __launch_bounds__(256) void paged_rows_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
@@ -1718,11 +1718,11 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
     });
 }
 
-// Merge of split rows, one workgroup per (token, head) row, with the optional
-// head sink folded in. Rows with a split count of 0 were written directly.
+// Merge of split rows with the optional head sink folded in. Rows with a split count of 0
+// were written directly.
 // One wave per row, two dims per lane: lane i weighs split i, and all of a row's loads go
 // out together. Bound by the partials' bytes: 1052 tokens of 32 heads of 128, 4 splits on
-// average, 31 us with a workgroup of two waves per row and one dim per thread.
+// average: 31 us with a workgroup of two waves per row and one dim per thread, 18 us now.
 constexpr int kMergeRows = 4;  // waves per workgroup
 template <typename T>
 __global__ __launch_bounds__(64 * kMergeRows) void paged_merge_kernel(
@@ -2108,9 +2108,11 @@ extern "C" int ortmi_group_query_attention(
         ORTMI_REQUIRE(total_sequence_length <= past_cap,
                       "GroupQueryAttention: total_sequence_length exceeds the KV buffer capacity");
     // The generic kernels take what the matrix-core tiles do not: present tensors that are
-    // not 16-byte aligned, and head 96's decode steps that the fast kernel does not take
+    // not 16-byte aligned, head 96's decode steps that the fast kernel does not take
     // (unaligned tensors, more than 8 query heads per KV head, a rotary half that is not a
-    // multiple of 8).
+    // multiple of 8), and its shortest prompts, which a workgroup per row finishes before a
+    // tile has started (24 / 8 heads, 8 tokens 7.9 us against 9.8; 16 tokens 8.7 and 9.3; 32
+    // tokens 10.7 and 10.5).
     if (dtype == ORTMI_F16 || dtype == ORTMI_BF16) {
         const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
         const bool packed = key == nullptr;
@@ -2122,7 +2124,9 @@ extern "C" int ortmi_group_query_attention(
                           (!rotary || rotary_interleaved || rotary_half % 8 == 0) && a16(query) &&
                           a16(kk) && a16(vv) && a16(present_key) && a16(present_value) &&
                           (past_cap == 0 || (a16(past_key) && a16(past_value)));
-        const bool tiles = a16(present_key) && a16(present_value);
+        const bool tiles = a16(present_key) && a16(present_value) &&
+                           (head_size != 96 || vp + seq_len > 24 ||
+                            batch * seq_len * num_heads > 1024);
         const bool decode = seq_len == 1 && (fast || head_size == 96);
         if (decode ? !fast : !tiles)
             return ortmi_group_query_attention_ex(
@@ -2624,10 +2628,15 @@ static int run_paged(const void* query, const void* key, const void* value, void
     // multi-token tile owns (output, partials, split counts) and runs before the
     // tile kernel on the same stream: beside it, on a second stream, its
     // workgroups took the CUs the tile workgroups (a whole CU each) were waiting
-    // for, and the pair finished no sooner than in sequence.
+    // for, and the pair finished no sooner than in sequence. Groups of 3 query heads left
+    // their single tokens to the tiles before (32 sequences to 6000 keys, 24 / 8 heads of
+    // 128: 240 -> 136 us); with a negative scale, whose maximum this kernel would take of the
+    // unscaled scores, they still do. Groups of 6 and 7 gain nothing: a workgroup's
+    // instructions bind it (24 sequences, 12 / 2 heads of 128: 105 us, 124 here).
     bool dec = false;
     if constexpr (VHD == HD) {
-        dec = vcache && value && pow2 && (G == 1 || G == 2 || G == 4 || G == 8);
+        dec = vcache && value && pow2 &&
+              (G == 1 || G == 2 || G == 4 || G == 8 || (G == 3 && sc > 0.f));
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(mt, KV, ns), dim3(256), 0, st, tiles, count, cum,
                                past, pk, blk_shift, qrot, H, sc, sink ? sink32 : nullptr, chunk,
@@ -2637,6 +2646,7 @@ static int run_paged(const void* query, const void* key, const void* value, void
             switch (G) {
                 case 1: launch(paged_decode_kernel<T, HD, 1>); break;
                 case 2: launch(paged_decode_kernel<T, HD, 2>); break;
+                case 3: launch(paged_decode_kernel<T, HD, 3>); break;
                 case 4: launch(paged_decode_kernel<T, HD, 4>); break;
                 case 8: launch(paged_decode_kernel<T, HD, 8>); break;
                 default: dec = false;

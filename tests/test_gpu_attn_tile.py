@@ -13,6 +13,7 @@ import math
 
 import pytest
 import torch
+from test_gpu_ops import _run_paged
 
 pytestmark = pytest.mark.gpu
 U = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
@@ -141,3 +142,12 @@ def test_gqa_tile_head96_keeps_probabilities(ortmi):
     want = (torch.softmax(sc, -1) @ vd).transpose(0, 1).reshape(S, H * hd)
     err = (out.double().cpu()[0] - want).abs()
     assert (err <= 2.0 ** -11 * want.abs() + 1000 * 2.0 ** -19).all(), err.max().item()
+
+
+@pytest.mark.parametrize("H,KV", [(6, 2), (14, 2)])
+@pytest.mark.parametrize("d,new_max,interleaved", [(64, 1, 0), (128, 3, 1)])
+def test_paged_group_sizes(ortmi, oracle, H, KV, d, new_max, interleaved):
+    """Single tokens of 3 query heads per KV head (the decode kernel) and of 7 (the tiles),
+    beside chunks on the tiles; long pasts split the keys."""
+    _run_paged(ortmi, oracle, H, KV, d, nb=100 * 3, blk=16, batch=3, seed=H + d, new_max=new_max,
+               rope=True, interleaved=interleaved)
