@@ -2,9 +2,10 @@
 // batches of 4-bit weights, and every shape of 8-bit weights and of fp32 activations
 // (blocks of 32, 64 or 128).
 //
-// 4-bit weights with fp16 or bf16 activations are dequantised to the activation type
-// ((q - zp) * s, one rounding), the weights the prefill GEMM multiplies. In the other
-// forms no weight is rounded: the codes enter the matrix cores as whole numbers
+// 4-bit weights with fp16 or bf16 activations of more than one row are dequantised to the
+// activation type ((q - zp) * s, one rounding), the weights the prefill GEMM multiplies. In
+// the other forms, and for a single row (K past the GEMV's, whose weights are not rounded
+// either), no weight is rounded: the codes enter the matrix cores as whole numbers
 // (q - zp), exact in fp16 and (up to a power of two) in bf16, v_mfma 16x16x32 sums the
 // 32 products of one chunk in fp32, and the chunk's sum takes its block's scale in
 // fp32. fp32 activations are split into three bf16 pieces of 8 mantissa bits each,
@@ -44,16 +45,16 @@ __device__ __forceinline__ U32Pair swap32u(uint32_t x, uint32_t y) {
 template <typename T>
 constexpr int blk_pieces() { return sizeof(T) == 4 ? 3 : 1; }
 
-// Dequantised weights (one rounding to T) instead of whole codes.
+// Forms with dequantised weights (one rounding to T) instead of whole codes, at M > 1.
 template <typename T, int BITS>
 constexpr bool blk_scaled() { return sizeof(T) == 2 && BITS == 4; }
 
 // A code enters bf16 operands as (q - zp) times this power of two (exact), so that a
 // chunk's 32 products sum to no more than the largest activation: no overflow that
 // the scaled weights would not have had. fp16 sums cannot overflow fp32.
-template <typename T, int BITS>
+template <typename T, int BITS, bool SC>
 constexpr float blk_unit() {
-    if (std::is_same<T, half_t>::value || blk_scaled<T, BITS>()) return 1.f;
+    if (std::is_same<T, half_t>::value || SC) return 1.f;
     return BITS == 4 ? 1.f / 512.f : 1.f / 8192.f;
 }
 
@@ -110,19 +111,20 @@ __device__ __forceinline__ u32x4_t scaled_codes(uint32_t w, uint32_t zp, uint32_
     return r;
 }
 
-// 8 codes as the 8 operand halves (q - zp) * blk_unit, in order.
+// 8 codes as the 8 operand halves (q - zp) * blk_unit, in order; 4-bit codes of fp16 in the
+// pair order of scaled_codes.
 template <typename T, int BITS>
 __device__ __forceinline__ u32x4_t blk_codes(uint32_t w0, uint32_t w1, uint32_t zp) {
     u32x4_t r;
     if constexpr (std::is_same<T, half_t>::value) {
-        static_assert(BITS == 8, "4-bit fp16 weights are scaled");
         const half_t zo = __builtin_bit_cast(half_t, (uint16_t)(0x6400u | zp));
         const half2_t z2 = {zo, zo};
         const uint32_t w[2] = {w0, w1};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const uint32_t m = __builtin_amdgcn_perm(0x64646464u, w[j / 2],
-                                                     j % 2 ? 0x04030402u : 0x04010400u);
+            const uint32_t m = BITS == 4 ? ((w0 >> (4 * j)) & 0x000F000Fu) | 0x64006400u
+                                         : __builtin_amdgcn_perm(0x64646464u, w[j / 2],
+                                                                 j % 2 ? 0x04030402u : 0x04010400u);
             r[j] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, m) - z2);
         }
     } else if constexpr (BITS == 4) {
@@ -235,13 +237,13 @@ uint32_t blk_lds(int nb) {
 // bytes per column and step, are copied to LDS whole before the first step.
 //
 // Lane (column, g) then reads chunk 4s + g (4-bit) or half chunk 4s + g (8-bit) of its
-// column. Dequantised weights (blk_scaled) need no exchange: matrix step c takes word
+// column. Dequantised weights (SC) need no exchange: matrix step c takes word
 // c of every group's own chunk and the activations at the same k. Whole codes must be
 // summed a chunk at a time: row swaps (v_permlane16/32_swap) give every lane group
 // its eight codes of each chunk in turn, so that one matrix step covers exactly one
 // chunk and its sum can take one scale; the chunk's scale and zero point are spread
 // to all groups the same way.
-template <typename T, int BITS, int MT, int NT, int NW, bool SWI>
+template <typename T, int BITS, int MT, int NT, int NW, bool SWI, bool SC>
 __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
     const T* __restrict__ A, const uint8_t* __restrict__ B, const T* __restrict__ S,
     const uint8_t* __restrict__ Z, T* __restrict__ Y, int M, int N, int K, int nb, int bshift,
@@ -249,7 +251,6 @@ __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
     using Stage = BlkStage<T, BITS, MT, NT>;
     constexpr int CH = Stage::CH, P = blk_pieces<T>(), SUB = Stage::SUB, PPR = Stage::PPR,
                   AI = Stage::AI, KSTEP = Stage::KSTEP, KSUB = KSTEP / SUB;
-    constexpr bool SC = blk_scaled<T, BITS>();
     extern __shared__ uint4 blk_smem[];
     uint8_t* const smem = reinterpret_cast<uint8_t*>(blk_smem);
 
@@ -481,7 +482,7 @@ __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
 #pragma unroll
                     for (int i = 0; i < MT; ++i) acc[i][t] = blk_mfma<T>(ao[i][0], bo, acc[i][t]);
                 } else {
-                    constexpr float inv = 1.f / blk_unit<T, BITS>();
+                    constexpr float inv = 1.f / blk_unit<T, BITS, SC>();
                     float sc;
                     if constexpr (sizeof(T) == 4)
                         sc = __uint_as_float(sv[t][c]) * inv;
@@ -570,13 +571,13 @@ __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
 // A tile shape and its launch. LDS allows 160 KB per workgroup; a K whose scales do
 // not fit takes fewer columns, and past one column tile none (-1).
 constexpr uint32_t kBlkLds = 160 * 1024;
-template <typename T, int BITS, int MT, int NT, int NW, bool SWI>
+template <typename T, int BITS, int MT, int NT, int NW, bool SWI, bool SC>
 int launch_blk(const T* A, const uint8_t* B, const T* S, const uint8_t* Z, T* Y, int M, int N,
                int K, int nb, int bshift, hipStream_t st) {
     const int tiles_m = (M + 16 * MT - 1) / (16 * MT), tiles_n = (N + 16 * NT - 1) / (16 * NT);
     const uint32_t lds = blk_lds<T, BITS, MT, NT, NW>(nb);
     if ((long)tiles_m * tiles_n > 0x7fffffffL || lds > kBlkLds) return -1;
-    hipLaunchKernelGGL((mnb_blk_kernel<T, BITS, MT, NT, NW, SWI>), dim3(tiles_m * tiles_n),
+    hipLaunchKernelGGL((mnb_blk_kernel<T, BITS, MT, NT, NW, SWI, SC>), dim3(tiles_m * tiles_n),
                        dim3(64 * NW), lds, st, A, B, S, Z, Y, M, N, K, nb, bshift, tiles_m, tiles_n);
     return check_launch("mnb_blk");
 }
@@ -612,8 +613,9 @@ int mnb_blk(const T* A, const uint8_t* B, const T* S, const uint8_t* Z, T* Y, in
         int (*launch)(const T*, const uint8_t*, const T*, const uint8_t*, T*, int, int, int, int,
                       int, hipStream_t);
     };
+    constexpr bool SC = blk_scaled<T, BITS>();
 #define ORTMI_SHAPE(MT, NT, NW) \
-    {MT, NT, NW, blk_lds<T, BITS, MT, NT, NW>(nb), launch_blk<T, BITS, MT, NT, NW, SWI>}
+    {MT, NT, NW, blk_lds<T, BITS, MT, NT, NW>(nb), launch_blk<T, BITS, MT, NT, NW, SWI, SC>}
     const Shape shapes[] = {ORTMI_SHAPE(1, 1, 8), ORTMI_SHAPE(1, 2, 8), ORTMI_SHAPE(1, 4, 8),
                             ORTMI_SHAPE(2, 1, 8), ORTMI_SHAPE(2, 2, 8), ORTMI_SHAPE(2, 4, 8),
                             ORTMI_SHAPE(2, 2, 4), ORTMI_SHAPE(2, 4, 4)};
@@ -633,7 +635,19 @@ int mnb_blk(const T* A, const uint8_t* B, const T* S, const uint8_t* Z, T* Y, in
         const double cost = rounds * (92.0 + share * steps * step * (c.nt + (c.mt == 1 ? 0.0 : 0.5)));
         if (!best || cost < least) best = &c, least = cost;
     }
-    return best ? best->launch(A, B, S, Z, Y, M, N, K, nb, bshift, st) : -1;
+    if (!best) return -1;
+    if constexpr (SC && !SWI) {
+        // One row keeps its weights unrounded, as the GEMV does at smaller K. MI355X, 4096
+        // columns: bf16 K 14336 15.0 us (scaled weights 13.8, VALU tile product 1764), fp16 K
+        // 17920 18.2 us (17.3, 2278).
+        if (M == 1) {
+            auto* launch = best->nt == 1   ? launch_blk<T, BITS, 1, 1, 8, false, false>
+                           : best->nt == 2 ? launch_blk<T, BITS, 1, 2, 8, false, false>
+                                           : launch_blk<T, BITS, 1, 4, 8, false, false>;
+            return launch(A, B, S, Z, Y, M, N, K, nb, bshift, st);
+        }
+    }
+    return best->launch(A, B, S, Z, Y, M, N, K, nb, bshift, st);
 }
 
 #define ORTMI_BLK(T, BITS, SWI)                                                            \

@@ -87,3 +87,39 @@ def test_mnb_blk_fp32_extremes(ortmi, oracle):
     assert np.isnan(got[2]).all()
     w = W[:, 3]
     assert (got[1][w > 0] == np.inf).all() and (got[1][w < 0] == -np.inf).all()
+
+
+@pytest.mark.parametrize("dt,K,N,block,asym", [
+    ("bf16", 11008, 515, 32, True),
+    ("bf16", 14336, 4096, 32, False),
+    ("bf16", 10248, 9003, 128, True),   # more column tiles per workgroup, K inside a block
+    ("f16", 16416, 1030, 32, True),
+    ("f16", 20488, 9003, 64, False),
+])
+def test_mnb_blk_one_row_keeps_weights(ortmi, oracle, dt, K, N, block, asym):
+    """One row of 4-bit weights past the K of the GEMV rounds no weight: nearly every output
+    is the exact sum rounded once. An fp32 sum is off by about 2^-20 of the outputs' rms, so
+    that less than one in a hundred lies near enough to a tie of the fp16 rounding (one in a
+    thousand, bf16) to fall on its other side; weights rounded to the type would move one
+    output in three. None is further off than one rounding and the bound of the sums."""
+    import torch
+
+    tdt = {"f16": torch.float16, "bf16": torch.bfloat16}[dt]
+    rng = np.random.default_rng(K + N)
+    A, B, s, zp = _mnb_inputs(rng, 1, N, K, block, asym=asym)
+    dA, ds = dev(A, tdt), dev(s, tdt)
+    got = host(ortmi.matmul_nbits(dA, dev(B), ds, dev(zp) if zp is not None else None, K=K, N=N,
+                                  block_size=block))[0].astype(np.float64)
+    A, s = dA.double().cpu().numpy()[0], ds.float().cpu().numpy()
+    nb = -(-K // block)
+    pick = np.arange(N) if N < 2000 else np.r_[np.arange(0, N, 17), N - 1]
+    W = oracle.mnb_dequant(B[pick], s.reshape(N, nb)[pick].ravel(),
+                           None if zp is None else zp.reshape(N, -1)[pick].ravel(), pick.size, K, 4,
+                           block).astype(np.float64)
+    exact, got = W @ A, got[pick]
+    rounded = torch.from_numpy(exact).to(tdt).double().numpy()
+    assert (got != rounded).mean() < 0.03, f"{(got != rounded).mean():.3f} rounded otherwise"
+    ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt]
+    adds = 32 + (K + 31) // 32 + 8
+    bound = ulp * np.abs(exact) + 2.0 ** -24 * adds * (np.abs(W) @ np.abs(A)) + 1e-7
+    assert (np.abs(got - exact) <= bound).all()
