@@ -437,6 +437,57 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
         const LanePair pr = swap32(lsum);
         lsum = pr.a + pr.b;
     }
+    if constexpr (HD == 96) {
+        // A value that is not finite must neither reach a row that does not see its key
+        // (through 0 * infinity) nor turn NaN between the pieces of P: the kernel that took
+        // these prompts before read visible keys only, in fp32. Every such product leaves a
+        // NaN in O; a wave that ends with one adds up P V again, a key at a time (m and the
+        // sum of P stand, they do not depend on V).
+        float z = 0.f;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) z = fmaf(oT[d][e], 0.f, z);
+        if (__any(z != 0.f)) {
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) oT[d][e] = 0.f;
+            const int last = min(k1 - 1, t.qpos0 + qtok);
+            const float mref = m == -INFINITY ? 0.f : m;
+            for (int n = 0; n < steps * kKeys; ++n) {
+                const int j = block(n / kKeys) + n % kKeys;
+                if (!__any(j <= last)) break;
+                const T *kr = kd + (int64_t)j * HD + 8 * hh, *vr = vd + (int64_t)j * HD + 4 * hh;
+                float dot = 0.f;
+#pragma unroll
+                for (int s2 = 0; s2 < QS; ++s2) {
+                    const u32x4_t w = *reinterpret_cast<const u32x4_t*>(kr + 16 * s2);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        dot = fmaf(tile_lo<T>(qf[s2][i]), tile_lo<T>(w[i]), dot);
+                        dot = fmaf(tile_hi<T>(qf[s2][i]), tile_hi<T>(w[i]), dot);
+                    }
+                }
+                const LanePair pr = swap32(dot);
+                const float p = __builtin_amdgcn_exp2f(fmaf(pr.a + pr.b, sc2, -mref));
+                if (j > last) continue;
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int e4 = 0; e4 < 4; ++e4) {
+                        const u32x2_t w =
+                            *reinterpret_cast<const u32x2_t*>(vr + 32 * d + 8 * e4);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            const int e = 4 * e4 + 2 * i;
+                            oT[d][e] = fmaf(p, tile_lo<T>(w[i]), oT[d][e]);
+                            oT[d][e + 1] = fmaf(p, tile_hi<T>(w[i]), oT[d][e + 1]);
+                        }
+                    }
+            }
+        }
+    }
 
     // --- the key groups' states, merged by the first (which alone has a single block) ----
     if (nblocks <= 1) {

@@ -126,6 +126,39 @@ def test_gqa_f32_tile_infinite_value_stays_in_its_rows(ortmi):
     assert torch.isfinite(out).all()
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
+@pytest.mark.parametrize("S,past,H,KV,at", [
+    (45, 0, 2, 2, 20),     # one block
+    (128, 0, 4, 4, 120),   # hidden to whole waves of the tile
+    (100, 70, 6, 2, 3),    # 42 tokens to a tile, a block that holds cached keys too
+    (40, 1500, 2, 1, 39),  # key splits
+])
+def test_gqa_tile_head96_value_stays_in_its_rows(ortmi, dt, value, S, past, H, KV, at):
+    """A value of a new token that is not finite reaches the rows of head 96 that see the
+    token, in its dim, and no other; the finite outputs are those of finite values."""
+    hd, tdt = 96, DT[dt]
+    g = torch.Generator().manual_seed(S + past)
+
+    def rnd(*shape):
+        return torch.randn(shape, generator=g).to(tdt).cuda()
+
+    q, k, v = rnd(1, S, H * hd), rnd(1, S, KV * hd), rnd(1, S, KV * hd)
+    pk, pv = rnd(1, KV, past, hd), rnd(1, KV, past, hd)
+    kw = dict(num_heads=H, kv_num_heads=KV)
+    want, _, _ = ortmi.group_query_attention(q, k, v, pk, pv, None, past + S, None, None, **kw)
+    v[0, at, 3] = value  # of KV head 0
+    out, _, _ = ortmi.group_query_attention(q, k, v, pk, pv, None, past + S, None, None, **kw)
+    out, want = (x.cpu()[0].reshape(S, H, hd) for x in (out, want))
+    hit = torch.zeros((S, H, hd), dtype=torch.bool)
+    hit[at:, :H // KV, 3] = True
+    bad = out[hit].double()
+    assert (torch.isnan(bad) if math.isnan(value) else bad == value).all()
+    # The block's sums run in another order: fp32 accumulation, and one rounding.
+    torch.testing.assert_close(out[~hit].double(), want[~hit].double(), rtol=2 * U[dt],
+                               atol=2.0 ** -16)
+
+
 def test_gqa_tile_head96_keeps_probabilities(ortmi):
     """Head 96 rounds no probability: with large values that cancel, the error stays at that
     of fp32 arithmetic and one rounding of the output."""
