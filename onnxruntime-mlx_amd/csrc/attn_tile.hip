@@ -96,8 +96,10 @@ constexpr int kRowWaves = kAttnRows / 32;  // waves of 32 query rows
 constexpr int kKeyGroups = 2;   // groups of waves that share the key blocks
 constexpr int kThreads = 64 * kRowWaves * kKeyGroups;
 
-// Pieces of P in the second product. Head 96 keeps its probabilities at fp32 precision,
-// as the kernel that took it before did: two fp16 pieces (22 bits) or three bf16 pieces.
+// Pieces of P in the second product. The kernel that took head 96 before had fp32
+// probabilities: three bf16 pieces carry their 24 bits, two fp16 pieces 22 bits down to 2^-17
+// of a row's largest and below that an error of 2^-39 of it (less than the error of the
+// exponential, a few 2^-22, down to 2^-18).
 template <typename T, int HD>
 constexpr int p_pieces() { return HD != 96 ? 1 : std::is_same<T, half_t>::value ? 2 : 3; }
 
@@ -373,10 +375,13 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
         // The reference point m moves only when the block max passes it by more than kLazy
         // (log2 units), so P = exp2(s - m) stays below 2^kLazy (exact in fp16's range) and
         // O is rarely rescaled; neither the final O / l nor a merge of (m, l, O) states
-        // depends on where m sits.
-        constexpr float kLazy = 8.f;
+        // depends on where m sits. With P in two fp16 pieces it sits 14 below the maximum and
+        // follows it closely: the second piece is subnormal, its error 2^-25, from P = 2^-3
+        // down, which is 2^-17 of the largest probability or less.
+        constexpr bool two16 = P == 2;
+        constexpr float kLazy = two16 ? 15.f : 8.f, kBelow = two16 ? 14.f : 0.f;
         const float bm = bmax * sc2;
-        const float m_new = bm > m + kLazy ? bm : m;
+        const float m_new = bm > m + kLazy ? bm - kBelow : m;
         // v_exp_f32 directly: results below 2^-126 flush to zero, which the softmax weights
         // can afford.
         const float alpha = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m - m_new);

@@ -177,6 +177,33 @@ def test_gqa_tile_head96_keeps_probabilities(ortmi):
     assert (err <= 2.0 ** -11 * want.abs() + 1000 * 2.0 ** -19).all(), err.max().item()
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("nats", [9.0, 12.0])
+def test_gqa_tile_head96_keeps_small_probabilities(ortmi, dt, nats):
+    """Probabilities of e^-9 and e^-12 beside one near 1 (whose value is 0) keep their bits:
+    large values that cancel leave the fp32 errors of the exponential, its argument (up to 16:
+    2^-21 of P each) and the sums, and the output's rounding."""
+    S, H, hd, tdt = 64, 2, 96, DT[dt]
+    g = torch.Generator().manual_seed(11)
+    q, k = (torch.randn((1, S, H, hd), generator=g) * 0.1 for _ in range(2))
+    q[..., 0] = math.sqrt(nats * math.sqrt(hd))
+    k[..., 0] = 0
+    k[:, 0, :, 0] = q[0, 0, 0, 0]
+    v = torch.full((1, S, H, hd), 30000.0)
+    v[:, 1::2] *= -1
+    v[:, 0] = 0
+    q, k, v = (x.to(tdt).reshape(1, S, H * hd) for x in (q, k, v))
+    z = torch.zeros((1, H, 0, hd), dtype=tdt, device="cuda")
+    out, _, _ = ortmi.group_query_attention(q.cuda(), k.cuda(), v.cuda(), z, z, None, S, None, None,
+                                            num_heads=H, kv_num_heads=H)
+    qd, kd, vd = (x.double().reshape(S, H, hd).transpose(0, 1) for x in (q, k, v))
+    sc = (qd @ kd.transpose(-1, -2)) / math.sqrt(hd)
+    p = torch.softmax(sc.masked_fill(torch.ones(S, S).triu(1).bool(), -math.inf), -1)
+    want, mag = ((p @ x).transpose(0, 1).reshape(S, H * hd) for x in (vd, vd.abs()))
+    excess = (out.double().cpu()[0] - want).abs() - U[dt] * want.abs() - 2.0 ** -20 * mag
+    assert excess.max().item() <= 0, excess.max().item()
+
+
 @pytest.mark.parametrize("H,KV", [(6, 2), (14, 2)])
 @pytest.mark.parametrize("d,new_max,interleaved", [(64, 1, 0), (128, 3, 1)])
 def test_paged_group_sizes(ortmi, oracle, H, KV, d, new_max, interleaved):
