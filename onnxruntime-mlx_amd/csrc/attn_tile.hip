@@ -2,8 +2,9 @@
 //
 // One workgroup of 8 waves takes 128 query rows of one KV head: 4 row waves of 32 rows,
 // twice, the two halves of the waves ("key groups") taking every other block of 64
-// keys; the groups' states are merged through LDS at the end. Everything a query needs
-// stays in its lanes:
+// keys; the groups' states are merged through LDS at the end. (A call whose keys all lie in
+// one block has workgroups of 4 waves, one group.) Everything a query needs stays in its
+// lanes:
 //   S^T = K Q^T     (v_mfma 32x32x16; A = 32 keys x 16 dims from LDS, B = 16 dims x 32
 //                    queries, held in registers for the whole tile)
 //   O^T += V^T P^T  (A = 32 head dims x 16 keys, B = this lane's own probabilities)
@@ -93,8 +94,7 @@ struct TileDesc {
 
 constexpr int kKeys = 64;       // keys per block
 constexpr int kRowWaves = kAttnRows / 32;  // waves of 32 query rows
-constexpr int kKeyGroups = 2;   // groups of waves that share the key blocks
-constexpr int kThreads = 64 * kRowWaves * kKeyGroups;
+// KG: groups of waves that share the key blocks, 1 or 2.
 
 // Pieces of P in the second product. The kernel that took head 96 before had fp32
 // probabilities: three bf16 pieces carry their 24 bits, two fp16 pieces 22 bits down to 2^-17
@@ -113,7 +113,7 @@ __device__ __forceinline__ int swizzle(int r) {
     return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
 }
 
-template <typename T, int HD>
+template <typename T, int HD, int KG>
 __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryRows<T>& qr,
                           const T* __restrict__ kd, const T* __restrict__ vd,
                           float scale, int k0, int k1,
@@ -126,10 +126,10 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
     constexpr int P = p_pieces<T, HD>();
     // Two buffers of K and V blocks per key group, arrays of their own so that a read of
     // one is known not to wait for the load in flight into the other.
-    __shared__ __attribute__((aligned(1024))) uint16_t sK0[kKeyGroups][kKeys * KC * 8];
-    __shared__ __attribute__((aligned(1024))) uint16_t sK1[kKeyGroups][kKeys * KC * 8];
-    __shared__ __attribute__((aligned(1024))) uint16_t sV0[kKeyGroups][kKeys * KC * 8];
-    __shared__ __attribute__((aligned(1024))) uint16_t sV1[kKeyGroups][kKeys * KC * 8];
+    __shared__ __attribute__((aligned(1024))) uint16_t sK0[KG][kKeys * KC * 8];
+    __shared__ __attribute__((aligned(1024))) uint16_t sK1[KG][kKeys * KC * 8];
+    __shared__ __attribute__((aligned(1024))) uint16_t sV0[KG][kKeys * KC * 8];
+    __shared__ __attribute__((aligned(1024))) uint16_t sV1[KG][kKeys * KC * 8];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int rw = wave % kRowWaves, kg = wave / kRowWaves;
@@ -170,7 +170,7 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
         return x;
     };
     const int per_load = 64 / KC;  // rows
-    auto load_rows = [&](uint16_t (&buf)[kKeyGroups][kKeys * KC * 8], const T* base, int kb) {
+    auto load_rows = [&](uint16_t (&buf)[KG][kKeys * KC * 8], const T* base, int kb) {
         const uint32_t ln = (uint32_t)opaque(lane);
         const int r0 = (int)(ln / KC), x = (int)(ln % KC) ^ swizzle<KC>(r0);
         int past_end = 0;
@@ -191,14 +191,14 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
         return past_end;
     };
     int vbad = 0;  // rows of the V block in flight that are to be zeroed
-    auto stage_k = [&](uint16_t (&buf)[kKeyGroups][kKeys * KC * 8], int kb) {
+    auto stage_k = [&](uint16_t (&buf)[KG][kKeys * KC * 8], int kb) {
         if (kb < k1) load_rows(buf, kd, kb);
     };
-    auto stage_v = [&](uint16_t (&buf)[kKeyGroups][kKeys * KC * 8], int kb) {
+    auto stage_v = [&](uint16_t (&buf)[KG][kKeys * KC * 8], int kb) {
         if (kb < k1) vbad = load_rows(buf, vd, kb);
     };
     // Waits for this wave's loads and zeroes the value rows that are not there.
-    auto arrive = [&](uint16_t (&buf)[kKeyGroups][kKeys * KC * 8]) {
+    auto arrive = [&](uint16_t (&buf)[KG][kKeys * KC * 8]) {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
         if (__any(vbad)) {
             const int ln = opaque(lane);
@@ -213,8 +213,8 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
 
     // Blocks of this group: k0 + (2 s + kg) * 64 in step s.
     const int nblocks = k1 > k0 ? (k1 - k0 + kKeys - 1) / kKeys : 0;
-    const int steps = (nblocks + kKeyGroups - 1) / kKeyGroups;
-    auto block = [&](int s) { return k0 + (kKeyGroups * s + kg) * kKeys; };
+    const int steps = (nblocks + KG - 1) / KG;
+    auto block = [&](int s) { return k0 + (KG * s + kg) * kKeys; };
     // --- queries ------------------------------------------------------------------
     // B operand of step s2: dims 16 s2 + 8 hh .. + 7 of the lane's query, rotated here
     // (one rounding to T) when the call has not staged rotated rows. Their loads go out
@@ -289,7 +289,7 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
 
     // --- the two products ---------------------------------------------------------
     const int kx0 = hh ^ swizzle<KC>(lrow);  // piece 2 s2 + hh of row lrow lies at kx ^ 2 s2
-    auto key_operand = [&](const uint16_t (&buf)[kKeyGroups][kKeys * KC * 8], int kx, int s2,
+    auto key_operand = [&](const uint16_t (&buf)[KG][kKeys * KC * 8], int kx, int s2,
                            int kt) {
         return *reinterpret_cast<const u32x4_t*>(&buf[kg][(kt * 32 * KC + (kx ^ (2 * s2))) * 8]);
     };
@@ -303,7 +303,7 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
         return (r * KC + (vlow ^ swizzle<KC>(r))) * 8 + 4 * (lane & 1);
     };
     const int v0 = voff(0), v1 = voff(1);
-    auto value_operand = [&](const uint16_t (&buf)[kKeyGroups][kKeys * KC * 8], int o0, int o1,
+    auto value_operand = [&](const uint16_t (&buf)[KG][kKeys * KC * 8], int o0, int o1,
                              int kk, int d) {
         const uint16_t* b = &buf[kg][kk * 16 * KC * 8];
         const u32x2_t lo = __builtin_bit_cast(
@@ -321,7 +321,7 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
     // the walk is bound by the instructions issued (interleaving both kinds inside a wave,
     // by halves of a block, issued more of them: 61 -> 66 us at 2048 tokens, 32 heads).
     float16_t stA[2], stB[2];
-    auto scores = [&](const uint16_t (&buf)[kKeyGroups][kKeys * KC * 8], float16_t (&st)[2]) {
+    auto scores = [&](const uint16_t (&buf)[KG][kKeys * KC * 8], float16_t (&st)[2]) {
         const int kx = opaque(lrow * KC + kx0);
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
@@ -334,10 +334,10 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
                 st[kt] = tile_mfma<T>(key_operand(buf, kx, s2, kt), qf[s2], st[kt]);
     };
     auto step = [&](int s, float16_t (&cur)[2], float16_t (&nxt)[2],
-                    uint16_t (&kfill)[kKeyGroups][kKeys * KC * 8],
-                    uint16_t (&knext)[kKeyGroups][kKeys * KC * 8],
-                    uint16_t (&vcur)[kKeyGroups][kKeys * KC * 8],
-                    uint16_t (&vfill)[kKeyGroups][kKeys * KC * 8]) {
+                    uint16_t (&kfill)[KG][kKeys * KC * 8],
+                    uint16_t (&knext)[KG][kKeys * KC * 8],
+                    uint16_t (&vcur)[KG][kKeys * KC * 8],
+                    uint16_t (&vfill)[KG][kKeys * KC * 8]) {
         const int kb = block(s);
         arrive(vcur);
         __syncthreads();
@@ -495,7 +495,7 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
     }
 
     // --- the key groups' states, merged by the first (which alone has a single block) ----
-    if (nblocks <= 1) {
+    if (KG == 1 || nblocks <= 1) {
         if (kg == 1 || !qlive) return;
     } else {
         constexpr int DK = KC / 8;  // head-dim tiles per K buffer pair (16 KB each)
@@ -563,8 +563,8 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
 // Grid B * KV * tiles * nsplit, the (sequence, KV head) fastest: with a multiple of 8 of
 // them the tiles that read the same keys run on one XCD. Tiles of later tokens, which
 // walk more keys, come first, so that the short ones fill the last round.
-template <typename T, int HD>
-__global__ __launch_bounds__(kThreads, 1) void gqa_tile_kernel(
+template <typename T, int HD, int KG>
+__global__ __launch_bounds__(64 * kRowWaves * KG, 1) void gqa_tile_kernel(
     QueryRows<T> q, const T* __restrict__ k, const T* __restrict__ v, int64_t cap, int B, int S,
     int QT, int tiles, int G, int H, int KV, int vp, float scale, T* __restrict__ out, int chunk,
     int nsplit, float* __restrict__ part, int* __restrict__ nsplit_row) {
@@ -589,8 +589,8 @@ __global__ __launch_bounds__(kThreads, 1) void gqa_tile_kernel(
     const int64_t slab = (int64_t)bkv * cap * HD;
     const int k0 = split * chunk;
     const int ks1 = split == ns - 1 ? k1 : min(k1, k0 + chunk);
-    attn_tile<T, HD>(t, kvh, G, H, q, k + slab, v + slab, scale, k0, ks1, out, (int64_t)H * HD,
-                     ns > 1 ? part : nullptr, nsplit, split);
+    attn_tile<T, HD, KG>(t, kvh, G, H, q, k + slab, v + slab, scale, k0, ks1, out, (int64_t)H * HD,
+                         ns > 1 ? part : nullptr, nsplit, split);
 }
 
 }  // namespace
@@ -602,14 +602,23 @@ int gqa_tile(const QueryRows<T>& q, const T* k, const T* v, int64_t cap, int B, 
     const int G = H / KV, QT = std::max(1, kAttnRows / G), tiles = (S + QT - 1) / QT;
     const int64_t grid = (int64_t)B * KV * tiles * nsplit;
     if (grid > 0x7fffffffLL) return fail(ORTMI_E_INVALID, "GroupQueryAttention: grid too large");
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kThreads), 0, st, q, k, v, cap, B, S,
-                           QT, tiles, G, H, KV, vp, scale, out, chunk, nsplit, part, nsplit_row);
+    auto launch = [&](auto kernel, int kg) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * kRowWaves * kg), 0, st, q, k, v,
+                           cap, B, S, QT, tiles, G, H, KV, vp, scale, out, chunk, nsplit, part,
+                           nsplit_row);
         return check_launch("gqa_tile");
     };
-    if (hd == 64) return launch(gqa_tile_kernel<T, 64>);
-    if (hd == 96) return launch(gqa_tile_kernel<T, 96>);
-    return launch(gqa_tile_kernel<T, 128>);
+    // All keys in one block: a second key group would have no work, and its waves and LDS
+    // would only lengthen the start. 32 heads of 128 on 8, 8, 32 and 64 tokens: 9.6, 12.0, 12.1
+    // us with two groups, 9.2, 11.1, 11.2 with one; 32 heads on 32, 32 tokens: 10.2 and 9.6.
+    if (vp + S <= kKeys) {
+        if (hd == 64) return launch(gqa_tile_kernel<T, 64, 1>, 1);
+        if (hd == 96) return launch(gqa_tile_kernel<T, 96, 1>, 1);
+        return launch(gqa_tile_kernel<T, 128, 1>, 1);
+    }
+    if (hd == 64) return launch(gqa_tile_kernel<T, 64, 2>, 2);
+    if (hd == 96) return launch(gqa_tile_kernel<T, 96, 2>, 2);
+    return launch(gqa_tile_kernel<T, 128, 2>, 2);
 }
 
 #define ORTMI_GQA_TILE(T)                                                                        \

@@ -102,6 +102,18 @@ def test_gqa_tile(ortmi, dt, hd, B, S, past, H, KV):
 
 
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("hd", [64, 96, 128])
+@pytest.mark.parametrize("B,S,past,H,KV", [
+    (2, 64, 0, 8, 2),     # one block of keys, full; two tiles
+    (1, 31, 33, 12, 2),   # cached keys in it
+    (9, 17, 0, 16, 16),   # a workgroup per head, ragged rows and keys
+])
+def test_gqa_tile_one_block(ortmi, dt, hd, B, S, past, H, KV):
+    """All keys in one block: tiles of one key group."""
+    check(ortmi, dt, B, S, past, H, KV, hd)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("opt", [
     dict(interleaved=True), dict(half=0), dict(half=16), dict(half=24, interleaved=True),
     dict(shared=False), dict(shift=1), dict(shift=3, interleaved=True), dict(scale=-0.2),
