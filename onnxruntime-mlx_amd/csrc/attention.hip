@@ -2015,7 +2015,7 @@ static int run_gqa(const void* query, const void* key, const void* value, const 
     // Rotary dims that fill the head, on 16-byte pieces, are rotated by the tile kernel as
     // it loads the queries; otherwise the prep kernel stages rotated queries.
     const bool pieces = (!cos_c || 2 * half == hd) && a16(q) && a16(k) && a16(v) && a16(cos_c) &&
-                        a16(sin_c);
+                        a16(sin_c) && a16(pk) && a16(pv);
     QueryRows<T> rows{qrot, (int64_t)H * hd, nullptr, nullptr, interleaved};
     if (pieces) {
         rows = {q, q_stride, static_cast<const T*>(cos_c), static_cast<const T*>(sin_c),
@@ -2107,28 +2107,25 @@ extern "C" int ortmi_group_query_attention(
     if (shared_c)
         ORTMI_REQUIRE(total_sequence_length <= past_cap,
                       "GroupQueryAttention: total_sequence_length exceeds the KV buffer capacity");
-    // The generic kernels take what the matrix-core tiles do not: present tensors that are
-    // not 16-byte aligned, head 96's decode steps that the fast kernel does not take
-    // (unaligned tensors, more than 8 query heads per KV head, a rotary half that is not a
-    // multiple of 8), and its shortest prompts, which a workgroup per row finishes before a
-    // tile has started (24 / 8 heads, 8 tokens 7.9 us against 9.8; 16 tokens 8.7 and 9.3; 32
-    // tokens 10.7 and 10.5).
-    if (dtype == ORTMI_F16 || dtype == ORTMI_BF16) {
+    // The generic kernels take what the others do not at head 96: prompts with present tensors
+    // that are not 16-byte aligned, decode steps that the fast kernel does not take (unaligned
+    // tensors, more than 8 query heads per KV head, a rotary half that is not a multiple of 8),
+    // and the shortest prompts, which a workgroup per row finishes before a tile has started
+    // (24 / 8 heads, 8 tokens 7.9 us against 9.8; 16 tokens 8.7 and 9.3; 32 tokens 10.7 and
+    // 10.5).
+    if (head_size == 96 && (dtype == ORTMI_F16 || dtype == ORTMI_BF16)) {
         const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
         const bool packed = key == nullptr;
-        const int64_t hb = head_size * 2;
-        const void* kk = packed ? static_cast<const char*>(query) + num_heads * hb : key;
-        const void* vv = packed ? static_cast<const char*>(query) + (num_heads + kv_num_heads) * hb
+        const void* kk = packed ? static_cast<const char*>(query) + num_heads * 96 * 2 : key;
+        const void* vv = packed ? static_cast<const char*>(query) + (num_heads + kv_num_heads) * 96 * 2
                                 : value;
         const bool fast = num_heads / kv_num_heads <= 8 &&
                           (!rotary || rotary_interleaved || rotary_half % 8 == 0) && a16(query) &&
                           a16(kk) && a16(vv) && a16(present_key) && a16(present_value) &&
                           (past_cap == 0 || (a16(past_key) && a16(past_value)));
         const bool tiles = a16(present_key) && a16(present_value) &&
-                           (head_size != 96 || vp + seq_len > 24 ||
-                            batch * seq_len * num_heads > 1024);
-        const bool decode = seq_len == 1 && (fast || head_size == 96);
-        if (decode ? !fast : !tiles)
+                           (vp + seq_len > 24 || batch * seq_len * num_heads > 1024);
+        if (seq_len == 1 ? !fast : !tiles)
             return ortmi_group_query_attention_ex(
                 query, key, value, past_key, past_value, past_cap, total_sequence_length,
                 cos_cache, sin_cache, rotary_half, max_pos, nullptr, nullptr, 1e-6f, nullptr, 0, 0,

@@ -25,7 +25,7 @@ struct QueryRows {
 // Dense prefill over present [B, KV, cap, hd]: queries at positions vp + s, keys
 // [0, vp + s]. With nsplit > 1 the keys are cut in chunks of `chunk`; rows of more than
 // one chunk leave partials [row][nsplit][hd + 2] and their split count (0: written).
-// Tensors 16-byte aligned; hd 64, 96 or 128.
+// Queries 16-byte aligned; k and v too at hd 96, at any element at hd 64 and 128.
 template <typename T>
 int gqa_tile(const QueryRows<T>& q, const T* k, const T* v, int64_t cap, int B, int S, int H,
              int KV, int hd, int vp, float scale, T* out, int chunk, int nsplit, float* part,

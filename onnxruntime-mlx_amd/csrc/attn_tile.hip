@@ -34,6 +34,7 @@ namespace {
 
 typedef uint16_t u16x8_t __attribute__((ext_vector_type(8)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));  // at any element
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(1))) void global_void;
@@ -113,7 +114,7 @@ __device__ __forceinline__ int swizzle(int r) {
     return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
 }
 
-template <typename T, int HD, int KG>
+template <typename T, int HD, int KG, bool A16>
 __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryRows<T>& qr,
                           const T* __restrict__ kd, const T* __restrict__ vd,
                           float scale, int k0, int k1,
@@ -165,6 +166,7 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
     // Addresses are formed anew in each block (a few instructions) from a value that the
     // compiler cannot see through: kept across blocks for all loads and buffers they would
     // take over 40 registers, and a spilled register's reload waits for the row loads.
+    // Rows that are not 16-byte aligned pass through registers to the same places.
     auto opaque = [](int x) {
         asm volatile("" : "+v"(x));
         return x;
@@ -174,6 +176,7 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
         const uint32_t ln = (uint32_t)opaque(lane);
         const int r0 = (int)(ln / KC), x = (int)(ln % KC) ^ swizzle<KC>(r0);
         int past_end = 0;
+        u32x4_t w[A16 ? 1 : KI];
 #pragma unroll
         for (int i = 0; i < KI; ++i) {
             // The first row of a load is a multiple of 4 (of 8 at 8 pieces), so that
@@ -184,9 +187,17 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
             const int r = first + r0, rc = min(r, k1 - 1 - kb);
             // A uniform base and a 32-bit offset inside the block.
             const T* src = base + (int64_t)kb * HD + (uint32_t)(rc * HD + c * 8);
-            __builtin_amdgcn_global_load_lds((global_void*)(void*)src,
-                                             (lds_void*)&buf[kg][(rw * KI + i) * 512], 16, 0, 0);
+            if constexpr (A16)
+                __builtin_amdgcn_global_load_lds((global_void*)(void*)src,
+                                                 (lds_void*)&buf[kg][(rw * KI + i) * 512], 16, 0, 0);
+            else
+                w[i] = *reinterpret_cast<const u32x4_any_t*>(src);
             past_end |= (int)(r != rc) << i;
+        }
+        if constexpr (!A16) {
+#pragma unroll
+            for (int i = 0; i < KI; ++i)
+                *reinterpret_cast<u32x4_t*>(&buf[kg][(rw * KI + i) * 512 + ln * 8]) = w[i];
         }
         return past_end;
     };
@@ -563,7 +574,7 @@ __device__ void attn_tile(const TileDesc& t, int kvh, int G, int H, const QueryR
 // Grid B * KV * tiles * nsplit, the (sequence, KV head) fastest: with a multiple of 8 of
 // them the tiles that read the same keys run on one XCD. Tiles of later tokens, which
 // walk more keys, come first, so that the short ones fill the last round.
-template <typename T, int HD, int KG>
+template <typename T, int HD, int KG, bool A16>
 __global__ __launch_bounds__(64 * kRowWaves * KG, 1) void gqa_tile_kernel(
     QueryRows<T> q, const T* __restrict__ k, const T* __restrict__ v, int64_t cap, int B, int S,
     int QT, int tiles, int G, int H, int KV, int vp, float scale, T* __restrict__ out, int chunk,
@@ -589,8 +600,8 @@ __global__ __launch_bounds__(64 * kRowWaves * KG, 1) void gqa_tile_kernel(
     const int64_t slab = (int64_t)bkv * cap * HD;
     const int k0 = split * chunk;
     const int ks1 = split == ns - 1 ? k1 : min(k1, k0 + chunk);
-    attn_tile<T, HD, KG>(t, kvh, G, H, q, k + slab, v + slab, scale, k0, ks1, out, (int64_t)H * HD,
-                         ns > 1 ? part : nullptr, nsplit, split);
+    attn_tile<T, HD, KG, A16>(t, kvh, G, H, q, k + slab, v + slab, scale, k0, ks1, out,
+                              (int64_t)H * HD, ns > 1 ? part : nullptr, nsplit, split);
 }
 
 }  // namespace
@@ -608,17 +619,24 @@ int gqa_tile(const QueryRows<T>& q, const T* k, const T* v, int64_t cap, int B, 
                            nsplit_row);
         return check_launch("gqa_tile");
     };
+    // Present tensors that are not 16-byte aligned pass through registers: 2048 tokens, 32
+    // heads of 128 on 8, 101 us off by one element (a workgroup per query row 4380), 73 aligned.
+    if ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) {
+        if (hd == 64) return launch(gqa_tile_kernel<T, 64, 2, false>, 2);
+        if (hd == 128) return launch(gqa_tile_kernel<T, 128, 2, false>, 2);
+        return fail(ORTMI_E_INVALID, "GroupQueryAttention: unaligned present tensor");
+    }
     // All keys in one block: a second key group would have no work, and its waves and LDS
     // would only lengthen the start. 32 heads of 128 on 8, 8, 32 and 64 tokens: 9.6, 12.0, 12.1
     // us with two groups, 9.2, 11.1, 11.2 with one; 32 heads on 32, 32 tokens: 10.2 and 9.6.
     if (vp + S <= kKeys) {
-        if (hd == 64) return launch(gqa_tile_kernel<T, 64, 1>, 1);
-        if (hd == 96) return launch(gqa_tile_kernel<T, 96, 1>, 1);
-        return launch(gqa_tile_kernel<T, 128, 1>, 1);
+        if (hd == 64) return launch(gqa_tile_kernel<T, 64, 1, true>, 1);
+        if (hd == 96) return launch(gqa_tile_kernel<T, 96, 1, true>, 1);
+        return launch(gqa_tile_kernel<T, 128, 1, true>, 1);
     }
-    if (hd == 64) return launch(gqa_tile_kernel<T, 64, 2>, 2);
-    if (hd == 96) return launch(gqa_tile_kernel<T, 96, 2>, 2);
-    return launch(gqa_tile_kernel<T, 128, 2>, 2);
+    if (hd == 64) return launch(gqa_tile_kernel<T, 64, 2, true>, 2);
+    if (hd == 96) return launch(gqa_tile_kernel<T, 96, 2, true>, 2);
+    return launch(gqa_tile_kernel<T, 128, 2, true>, 2);
 }
 
 #define ORTMI_GQA_TILE(T)                                                                        \

@@ -123,6 +123,19 @@ def test_gqa_tile_options(ortmi, dt, hd, opt):
     check(ortmi, dt, 2, 37, 70, 8, 2, hd, **opt)
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("B,S,past,H,KV,opt", [
+    (1, 300, 0, 4, 4, dict(shift=1)),               # several blocks and tiles, the last ragged
+    (1, 5, 1500, 32, 8, dict(shift=7)),             # key splits
+    (2, 1, 70, 18, 2, dict(shift=4)),               # one token the decode kernel does not take
+    (2, 70, 33, 8, 2, dict(shift=5, shared=False)), # past rows copied from unaligned tensors
+])
+def test_gqa_tile_unaligned(ortmi, dt, hd, B, S, past, H, KV, opt):
+    """Tensors that start at any element: the tiles' rows pass through registers."""
+    check(ortmi, dt, B, S, past, H, KV, hd, **opt)
+
+
 def test_gqa_f32_tile_infinite_value_stays_in_its_rows(ortmi):
     """An infinite value of a key reaches the rows that see the key and no other."""
     S, H, hd = 45, 2, 64
