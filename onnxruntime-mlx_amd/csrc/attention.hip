@@ -519,7 +519,8 @@ __global__ __launch_bounds__(256) void gqa_decode_kernel(
 
     // 3. RoPE of the queries and of the new key. Scores are kept as raw dot
     // products of the rounded query with the keys; the softmax scale (and log2 e,
-    // for the hardware exp2) is applied inside the exponent.
+    // for the hardware exp2) is applied inside the exponent, which needs it positive:
+    // a negative scale turns the sign of the query.
     constexpr bool kDot2 = std::is_same<T, half_t>::value;
     float qf[G][8];
     half2_t q2[G][4];
@@ -557,7 +558,16 @@ __global__ __launch_bounds__(256) void gqa_decode_kernel(
         __builtin_memcpy(&knb, kt, sizeof(knb));
     }
     constexpr float kLog2e = 1.4426950408889634f;
-    const float c2 = scale * kLog2e;
+    const float c2 = fabsf(scale) * kLog2e;
+    if (scale < 0.f) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) qf[g][i] = -qf[g][i];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) q2[g][p] = -q2[g][p];
+        }
+    }
     // Partial dot product of a head's query with 8 dims of a key (this lane's).
     auto qk = [&](int g, const u32x4_t& kv) -> float {
         float d = 0.f;
@@ -665,7 +675,7 @@ __global__ __launch_bounds__(256) void gqa_decode_kernel(
     // Back to natural-log units for the merges (scores times the scale).
 #pragma unroll
     for (int g = 0; g < G; ++g)
-        if (m[g] != -INFINITY) m[g] *= scale;
+        if (m[g] != -INFINITY) m[g] *= fabsf(scale);
     // The new row (RoPE'd key, value) goes to row vp of the present buffer, from
     // the split that owns it; it is written last so no reload waits on it.
     {
@@ -1555,13 +1565,18 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
     const int bmask = (1 << blk_shift) - 1;
 
     // Scores are raw dot products with the rotated query; the softmax scale (and
-    // log2 e, for the hardware exp2) is applied inside the exponent. fp16 rows
+    // log2 e, for the hardware exp2) is applied inside the exponent, which needs it
+    // positive: a negative scale turns the sign of the query. fp16 rows
     // take two dims per v_dot2_f32_f16 (exact products, fp32 accumulation).
     constexpr bool kDot2 = std::is_same<T, half_t>::value;
+    const uint32_t qsign = scale < 0.f ? 0x80008000u : 0u;
     uint4 qraw[G];
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+    for (int g = 0; g < G; ++g) {
         qraw[g] = *reinterpret_cast<const uint4*>(qrot + ((int64_t)tok * H + kvh * G + g) * HD + dl);
+        qraw[g] = make_uint4(qraw[g].x ^ qsign, qraw[g].y ^ qsign, qraw[g].z ^ qsign,
+                             qraw[g].w ^ qsign);
+    }
     auto qk = [&](int g, const uint4& kv) -> float {
         float d = 0.f;
         if constexpr (kDot2) {
@@ -1580,7 +1595,7 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
         return d;
     };
     constexpr float kLog2e = 1.4426950408889634f;
-    const float c2 = scale * kLog2e;
+    const float c2 = fabsf(scale) * kLog2e;
     float m[G], l[G], o[G][8];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -1693,7 +1708,7 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
     // Back to natural-log units for the merges (scores times the scale).
 #pragma unroll
     for (int g = 0; g < G; ++g)
-        if (m[g] != -INFINITY) m[g] *= scale;
+        if (m[g] != -INFINITY) m[g] *= fabsf(scale);
 
     decode_merge<HD, G, LPR, 4>(m, l, o, s_m, s_l, s_o, [&](int g, int d, float M, float L, float acc) {
         const int h = kvh * G + g;
@@ -2627,13 +2642,11 @@ static int run_paged(const void* query, const void* key, const void* value, void
     // workgroups took the CUs the tile workgroups (a whole CU each) were waiting
     // for, and the pair finished no sooner than in sequence. Groups of 3 query heads left
     // their single tokens to the tiles before (32 sequences to 6000 keys, 24 / 8 heads of
-    // 128: 240 -> 136 us); with a negative scale, whose maximum this kernel would take of the
-    // unscaled scores, they still do. Groups of 6 and 7 gain nothing: a workgroup's
-    // instructions bind it (24 sequences, 12 / 2 heads of 128: 105 us, 124 here).
+    // 128: 240 -> 136 us). Groups of 6 and 7 gain nothing: a workgroup's instructions bind it
+    // (24 sequences, 12 / 2 heads of 128: 105 us, 124 here).
     bool dec = false;
     if constexpr (VHD == HD) {
-        dec = vcache && value && pow2 &&
-              (G == 1 || G == 2 || G == 4 || G == 8 || (G == 3 && sc > 0.f));
+        dec = vcache && value && pow2 && (G == 1 || G == 2 || G == 3 || G == 4 || G == 8);
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(mt, KV, ns), dim3(256), 0, st, tiles, count, cum,
                                past, pk, blk_shift, qrot, H, sc, sink ? sink32 : nullptr, chunk,

@@ -11,9 +11,10 @@ from __future__ import annotations
 
 import math
 
+import numpy as np
 import pytest
 import torch
-from test_gpu_ops import _run_paged
+from test_gpu_ops import _run_paged, assert_f16_close, dev, host
 
 pytestmark = pytest.mark.gpu
 U = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
@@ -236,3 +237,34 @@ def test_paged_group_sizes(ortmi, oracle, H, KV, d, new_max, interleaved):
     beside chunks on the tiles; long pasts split the keys."""
     _run_paged(ortmi, oracle, H, KV, d, nb=100 * 3, blk=16, batch=3, seed=H + d, new_max=new_max,
                rope=True, interleaved=interleaved)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("hd,H,KV", [(64, 8, 8), (96, 6, 2), (128, 8, 1)])
+@pytest.mark.parametrize("shared", [True, False])
+def test_gqa_one_token_negative_scale(ortmi, dt, hd, H, KV, shared):
+    """Scores of some +-100: the maximum that the exponents are taken from is that of the
+    scaled scores, not of the raw products."""
+    check(ortmi, dt, 2, 1, 300, H, KV, hd, half=0, scale=-4.0, shared=shared)
+
+
+@pytest.mark.parametrize("H,KV", [(2, 2), (4, 2), (6, 2), (8, 2), (8, 1), (7, 1)])
+def test_paged_one_token_negative_scale(ortmi, oracle, H, KV):
+    """The same over a paged cache, for each group size of the decode kernel and one of the
+    tiles; two sequences split their keys."""
+    rng = np.random.default_rng(H)
+    d, blk, batch, maxb = 64, 16, 3, 80
+    past = np.array([37, 700, 1279], np.int32)
+    cum = np.arange(batch + 1, dtype=np.int32)
+
+    def rnd(*shape):
+        return rng.standard_normal(shape).astype(np.float16)
+
+    q, k, v = rnd(batch, H * d), rnd(batch, KV * d), rnd(batch, KV * d)
+    kc, vc = rnd(maxb * batch, blk, KV, d), rnd(maxb * batch, blk, KV, d)
+    bt = rng.permutation(maxb * batch).astype(np.int32).reshape(batch, maxb)
+    out = ortmi.paged_attention(dev(q), dev(k), dev(v), dev(kc), dev(vc), dev(cum), dev(past),
+                                dev(bt), num_heads=H, kv_num_heads=KV, scale=-4.0)
+    want, _, _ = oracle.paged_attention(q, k, v, kc, vc, cum, past, bt, H, KV, scale=-4.0,
+                                        round16=True)
+    assert_f16_close(host(out), want, what="paged one token, scale -4")
