@@ -159,7 +159,8 @@ __device__ __forceinline__ u32x4_t blk_codes(uint32_t w0, uint32_t w1, uint32_t 
 // order; bf16 as is; fp32 as three bf16 pieces: the high 16 bits, the high 16 bits
 // of the exact remainder, and the rest (8 bits each). The remainder of an infinity
 // would be NaN: it is held to a finite value (below any overflow, above every real
-// remainder), so an infinity stays one.
+// remainder), so an infinity stays one, and a NaN without payload in its high half turns
+// into one (the kernel's end sees to those).
 template <typename T, int BITS>
 __device__ __forceinline__ void blk_acts(const u32x4_t* raw, u32x4_t* op) {
     if constexpr (sizeof(T) == 4) {
@@ -552,6 +553,15 @@ __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
 #pragma unroll
         for (int j = 0; j < NW; ++j) v += red[((j * MT * NT + it) * 4 + e) * 64 + lane];
         const int m = m0 + 16 * (it / NT) + 4 * g + e, n = n0 + 16 * (it % NT) + li;
+        if constexpr (sizeof(T) == 4) {
+            // A NaN whose payload lies in the low 16 bits alone entered as an infinity (its
+            // first piece), which left no finite sum: an infinite one looks for NaN in its row.
+            if (__builtin_isinf(v) && m < M)
+                for (int k = 0; k < K; ++k) {
+                    const float x = A[(size_t)m * K + k];
+                    if (x != x) v = x;
+                }
+        }
         if constexpr (SWI) {
             // Interleaved gate/up columns (2i, 2i + 1) in adjacent lanes: the even lane
             // writes column i of the [M, N / 2] output, (g * sigmoid(g)) * u with each

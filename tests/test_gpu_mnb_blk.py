@@ -123,3 +123,22 @@ def test_mnb_blk_one_row_keeps_weights(ortmi, oracle, dt, K, N, block, asym):
     adds = 32 + (K + 31) // 32 + 8
     bound = ulp * np.abs(exact) + 2.0 ** -24 * adds * (np.abs(W) @ np.abs(A)) + 1e-7
     assert (np.abs(got - exact) <= bound).all()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_mnb_blk_fp32_signalling_nan(ortmi, oracle, bits):
+    """A NaN whose payload lies in the low 16 bits alone gives NaN rows, not infinities."""
+    import torch
+
+    def edit(a):
+        words = a.view(torch.int32)
+        words[3, 7] = 0x7F800001
+        words[11, 200] = 0xFF80FFFF - (1 << 32)
+        a[5, 9] = float("inf")
+
+    with np.errstate(invalid="ignore"):
+        got, A, W = _run(ortmi, oracle, "f32", 20, 512, 96, bits, 32, True, edit)
+    assert np.isnan(A[3, 7]) and np.isnan(A[11, 200])
+    rows = [i for i in range(20) if i not in (3, 5, 11)]
+    assert np.isnan(got[[3, 11]]).all() and np.isfinite(got[rows]).all()
+    assert np.isinf(got[5][W[:, 9] != 0]).all()
