@@ -234,7 +234,7 @@ uint32_t blk_lds(int nb) {
 // cycle per lane (M = 2, 4096 x 14336, fp16: 19.0 us). So four neighbouring lanes
 // load 64 contiguous bytes (of a column; a whole row part of the activations), and
 // each wave passes what it loaded through an LDS region of its own (same-wave LDS
-// accesses stay in order: no barrier). The scales and zero points of the tile, a few
+// accesses stay in order: no workgroup barrier). The scales and zero points of the tile, a few
 // bytes per column and step, are copied to LDS whole before the first step.
 //
 // Lane (column, g) then reads chunk 4s + g (4-bit) or half chunk 4s + g (8-bit) of its
@@ -379,13 +379,22 @@ __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[i][t] = float4_t{0.f, 0.f, 0.f, 0.f};
 
+    // Between a wave's accesses of its region by one lane and those by another: the hardware
+    // keeps them in order, and this keeps the compiler from moving one past the other.
+    auto exchange = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+    };
+
     // Multiplies a stage; its registers take the loads of step `next` as soon as their
     // contents are in LDS.
     auto process = [&](Stage& st, int step, int next) {
+        exchange();
 #pragma unroll
         for (int t = 0; t < NT; ++t)
             *reinterpret_cast<u32x4_t*>(wreg + 1024 * t + b_put) = st.b[t];
         put_a(st, 0);
+        exchange();
         uint32_t w[NT][4];
         // Scale and zero point, of the lane's chunk (SC) or of each chunk.
         constexpr int NS = SC ? 1 : CH;
@@ -460,7 +469,9 @@ __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (SUB == 2) {
                 if (c == CH / 2) {
+                    exchange();
                     put_a(st, 1);
+                    exchange();
                     load(st, next);
                 }
             }
