@@ -243,6 +243,10 @@ int ortmi_decoder_decode_step(const OrtmiDecoderLayer* layers, const OrtmiDecode
  * cos_cache/sin_cache [max_pos, rotary_half] (NULL when do_rotary = 0), in dtype.
  * output [B,S,H*hd]. scale = 0 means 1/sqrt(hd). hd is 64, 96 or 128 (other head
  * sizes, fp32, attention_bias and QK-norm: ortmi_group_query_attention_ex).
+ * ortmi_group_query_attention_workspace_size gives the size for which a prompt of few
+ * rows over many keys is cut into as many key splits as pay (up to 16). A smaller
+ * workspace is taken too, down to the rotated queries, the one-token splits and two
+ * prompt splits; fewer splits sum in another order. Below that: ORTMI_E_WORKSPACE.
  * Replaces: group_query_attention_op (rust/src/ops/attention.rs:556-952): the
  * two mlx_fast_rope calls (attention.rs:671-708), the KV concat /
  * slice_update (attention.rs:881-908) and mlx_fast_scaled_dot_product_attention

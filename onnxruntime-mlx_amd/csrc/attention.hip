@@ -1901,9 +1901,11 @@ extern "C" size_t ortmi_group_query_attention_workspace_size(int64_t batch, int6
                                                              int64_t num_heads, int64_t head_size,
                                                              int64_t total_kv) {
     // As many splits as the call would use: whole CUs over the tiles these rows fill, of
-    // at least 512 keys each.
+    // at least 512 keys each. 256 CUs whatever the device (a partition has fewer and uses
+    // fewer splits), so that the size depends on the arguments alone.
+    constexpr int64_t kMaxCus = 256;
     const int64_t rows = std::max<int64_t>(1, batch * seq_len * num_heads);
-    const int64_t splits = std::min<int64_t>({(int64_t)kMaxPrefillSplits, 256 * kAttnRows / rows,
+    const int64_t splits = std::min<int64_t>({(int64_t)kMaxPrefillSplits, kMaxCus * kAttnRows / rows,
                                               (std::max<int64_t>(total_kv, 0) + 511) / 512});
     return gqa_workspace(batch, seq_len, num_heads, head_size, total_kv,
                          std::max<int64_t>(splits, kPrefillSplits));
@@ -2347,8 +2349,8 @@ extern "C" int ortmi_group_query_attention_noalloc(
                   "GroupQueryAttention: bad shape");
     int64_t vp = (int64_t)total_sequence_length - seq_len;
     if (vp < 0 || vp > past_cap) vp = past_cap;
-    const size_t need =
-        gqa_workspace(batch, seq_len, num_heads, head_size, vp + seq_len, kPrefillSplits);
+    const size_t need = ortmi_group_query_attention_workspace_size(batch, seq_len, num_heads,
+                                                                   head_size, vp + seq_len);
     if (need > kGqaScratchBytes)
         return fail(ORTMI_E_WORKSPACE,
                     "GroupQueryAttention (no-alloc): needs " + std::to_string(need) +

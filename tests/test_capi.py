@@ -83,3 +83,21 @@ def test_workspace_sizes_are_monotone(lib):
 
 def test_package_layout():
     assert os.path.isdir(os.path.join(PKG_DIR, "csrc"))
+
+
+def test_gqa_key_splits_fit_the_fixed_scratch(lib):
+    """The no-alloc entry refuses by the workspace size. Room for more than the two prompt
+    splits of the smallest workspace must not make it refuse a call that fits with two."""
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    for hd in (64, 96, 128):
+        for H in (1, 8, 32, 96):
+            for S in (2, 5, 37, 160, 600):
+                for total in (S, 1500, 9000):
+                    rows = S * H
+                    two = up(rows * hd * 4) + max(
+                        up(H * -(-total // 64) * (hd + 2) * 4),
+                        up(rows * 2 * (hd + 2) * 4) + up(rows * 4))
+                    size = lib.ortmi_group_query_attention_workspace_size(1, S, H, hd, total)
+                    assert size >= two
+                    scratch = lib.ortmi_group_query_attention_noalloc_max_workspace()
+                    assert size <= scratch or two > scratch or size == two

@@ -137,6 +137,33 @@ def test_gqa_tile_unaligned(ortmi, dt, hd, B, S, past, H, KV, opt):
     check(ortmi, dt, B, S, past, H, KV, hd, **opt)
 
 
+def test_gqa_tile_smallest_workspace(ortmi):
+    """The smallest workspace of a prompt has room for two key splits instead of four; less
+    is an error, and nothing is launched."""
+    S, H, KV, hd, past = 40, 32, 8, 128, 1500
+    lib = ortmi.load_kernels()
+    g = torch.Generator().manual_seed(9)
+    q, k, v, pk, pv = (torch.randn(n, generator=g).half().cuda() for n in (
+        (1, S, H * hd), (1, S, KV * hd), (1, S, KV * hd), (1, KV, past + S, hd),
+        (1, KV, past + S, hd)))
+    full = lib.ortmi_group_query_attention_workspace_size(1, S, H, hd, past + S)
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    least = up(S * H * hd * 4) + up(S * H * 2 * (hd + 2) * 4) + up(S * H * 4)
+    assert least < full
+    ws = torch.empty(full, dtype=torch.uint8, device="cuda")
+    outs = []
+    for size, status in ((full, 0), (least, 0), (least - 1, 3)):
+        out = torch.zeros_like(q)
+        rc = lib.ortmi_group_query_attention(
+            *(x.data_ptr() for x in (q, k, v, pk, pv)), past + S, past + S, None, None, 0, 0,
+            *(x.data_ptr() for x in (out, pk, pv)), 1, S, H, KV, hd, 0.0, 0, 10, ws.data_ptr(), size,
+            torch.cuda.current_stream().cuda_stream)
+        assert rc == status
+        outs.append(out.double().cpu())
+    assert_f16_close(outs[1].numpy(), outs[0].numpy(), what="two key splits")
+    assert outs[0].abs().max() > 0 and outs[2].abs().max() == 0
+
+
 def test_gqa_f32_tile_infinite_value_stays_in_its_rows(ortmi):
     """An infinite value of a key reaches the rows that see the key and no other."""
     S, H, hd = 45, 2, 64
