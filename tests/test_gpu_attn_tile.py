@@ -124,6 +124,14 @@ def test_gqa_tile_options(ortmi, dt, hd, opt):
     check(ortmi, dt, 2, 37, 70, 8, 2, hd, **opt)
 
 
+@pytest.mark.parametrize("opt", [dict(interleaved=True), dict(half=16), dict(shared=False),
+                                 dict(shift=1), dict(scale=-0.2), dict(packed=True)])
+@pytest.mark.parametrize("hd", [64, 96, 128])
+def test_gqa_f32_tile_options(ortmi, hd, opt):
+    """fp32: the sign branch, and the fallback for rows that are not 16-byte aligned."""
+    check(ortmi, "f32", 2, 37, 70, 8, 2, hd, **opt)
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("B,S,past,H,KV,opt", [
