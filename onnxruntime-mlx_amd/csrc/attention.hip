@@ -818,7 +818,7 @@ struct TileDesc {
 
 constexpr int kKeyTile = 64;
 
-// The attention tile on the matrix cores (fp16), 128 query rows per workgroup,
+// The attention tile on the matrix cores (fp16 and bf16), 256 query rows per workgroup,
 // computed transposed so that everything a query needs stays in its lanes:
 //   S^T = K Q^T     (v_mfma_f32_32x32x16_f16; A = 32 keys x 16 dims from LDS,
 //                    B = 16 dims x 32 queries, held in registers for the whole tile)
@@ -871,13 +871,14 @@ __device__ __forceinline__ float tile_pair_sum(uint32_t w, float acc) {
 
 template <typename T, int HD, int VHD, int NW>
 __device__ void attn_mfma_body(const TileDesc& t, int kvh, int G, int H,
-                               const T* __restrict__ qrot, const PagedKV& pk, float scale, const float* __restrict__ sink,
-                               int k0, int k1, T* __restrict__ out, int64_t out_tok_stride,
+                               const T* __restrict__ qrot, const PagedKV& pk, float scale,
+                               const float* __restrict__ sink, int k0, int k1,
+                               T* __restrict__ out, int64_t out_tok_stride,
                                float* __restrict__ part, int nsplit, int split) {
     static_assert(std::is_same<T, half_t>::value || std::is_same<T, uint16_t>::value,
                   "fp16 or bf16 (16-bit storage)");
     static_assert(kKeyTile == 64 && HD % 16 == 0 && VHD % 32 == 0, "tile shape");
-    static_assert(NW == 4 || NW == 8, "waves per tile");
+    static_assert(NW == 8, "waves per tile");
     constexpr int NT = 64 * NW;       // threads
     constexpr int kRows = 32 * NW;    // query rows of the tile (32 per wave)
     constexpr int KP = HD + 8, VP = kKeyTile + 8;
