@@ -249,6 +249,8 @@ def test_mnb_gemv_fp16_interleaved_symmetric(ortmi, oracle, K, N):
 @pytest.mark.parametrize("K,N,block", [(256, 192, 32), (512, 256, 64), (384, 160, 128),
                                        (1176, 64, 32)])
 def test_mnb_gemm_fp16(ortmi, oracle, M, K, N, block):
+    """Small fp16 products: all of them, being below 65 rows or 2^20 outputs, on the kernel
+    that splits K over waves (the prefill GEMM: test_mnb_gemm_forms)."""
     rng = np.random.default_rng(M * 11 + K + N + block)
     A, B, s, zp = _mnb_inputs(rng, M, N, K, block, dtype=np.float16)
     got = host(ortmi.matmul_nbits(dev(A), dev(B), dev(s), dev(zp), K=K, N=N, block_size=block))
@@ -278,7 +280,7 @@ def _check_gemm_rows(oracle, got_rows, A_rows, B, s, zp, N, K, block, what):
 
 @pytest.mark.parametrize("M,N,K", [
     (512, 4096, 4096),   # the prefill GEMM config
-    (512, 1536, 8960),   # the decoder prefill's down_proj (64x64 tiles, k split)
+    (512, 1536, 8960),   # the decoder prefill's down_proj (K split over waves)
     (512, 2048, 1536),   # the decoder prefill's merged QKV
 ])
 def test_mnb_gemm_config2_shape(ortmi, oracle, M, N, K):
@@ -303,13 +305,42 @@ def test_mnb_gemm_large_tiles(ortmi, oracle, M, N, K, block):
     _check_gemm_rows(oracle, got[rows], A[rows], B, s, zp, N, K, block, "gemm large tiles")
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("block", [32, 64, 128])
+@pytest.mark.parametrize("M,N", [(515, 2050), (515, 4100), (1030, 8200)])
+def test_mnb_gemm_forms(ortmi, oracle, dt, block, M, N):
+    """The prefill GEMM in both types: 64x64 and 64x128 tiles (k-steps split over two wave
+    groups) and 128x128 tiles (weights in registers), ragged in M, N and K. Against 64-bit
+    A . W^T with the weights rounded to the type once, as the kernel feeds them: the output's
+    rounding and fp32 accumulation over 1000 products (2^-24 each, worst case)."""
+    import torch
+
+    K, tdt = 1000, {"f16": torch.float16, "bf16": torch.bfloat16}[dt]
+    rng = np.random.default_rng(M + N + block)
+    A, B, s, zp = _mnb_inputs(rng, M, N, K, block)
+    dA, ds = dev(A, tdt), dev(s, tdt)
+    got = host(ortmi.matmul_nbits(dA, dev(B), ds, dev(zp), K=K, N=N, block_size=block))
+    rows = np.r_[np.arange(0, M, 41), M - 1]
+    A, s = dA.double().cpu().numpy()[rows], ds.float().cpu().numpy()
+    W = refs.dequant_ref(B, s, zp, N, K, 4, block).astype(np.float32)
+    W = torch.from_numpy(W).to(tdt).double().numpy()
+    want = A @ W.T
+    u = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt]
+    bound = u * np.abs(want) + 2.0 ** -24 * K * (np.abs(A) @ np.abs(W).T)
+    excess = np.abs(got[rows] - want) - bound
+    assert excess.max() <= 0, f"max excess {excess.max():.3e}"
+
+
 @pytest.mark.parametrize("M,N,K,block", [(37, 400, 1536, 32), (512, 2048, 1536, 32),
-                                         (512, 17920, 1536, 32), (64, 256, 1000, 64)])
+                                         (512, 17920, 1536, 32), (64, 256, 1000, 64),
+                                         (515, 2050, 1000, 64), (515, 4100, 1000, 128),
+                                         (1030, 8200, 1000, 32)])
 def test_mnb_gemm_swiglu_pairs(ortmi, oracle, M, N, K, block):
     """SwiGLU in the GEMM epilogue over interleaved gate/up rows equals the GEMM
     followed by the SwiGLU-pairs kernel bit for bit (the same tile walk), and the
     oracle's unfused ops (fp16 matmul outputs, SwiGLU op by op) within tolerance.
-    The shapes cover the 64x64, 64x128 and 128x128 tile forms and K % 64 != 0."""
+    The shapes cover the kernel that splits K over waves (37 and 64 rows) and the GEMM's
+    64x64, 64x128 and 128x128 tile forms, each with K % 64 != 0."""
     import ctypes
 
     import torch
@@ -371,8 +402,8 @@ def test_mnb_bf16(ortmi, oracle, M, K, N, block, asym):
                                          (40, 1024, 384, 64), (96, 768, 200, 128),
                                          (512, 4096, 4096, 32)])
 def test_mnb_gemm_bf16(ortmi, oracle, M, K, N, block):
-    """bf16 prefill on the matrix cores (v_mfma_f32_32x32x16_bf16), zero points
-    U{0..15}. Primary check: against fp64 A . Wbf16^T with the dequantised weights
+    """bf16 prompts on the matrix cores (512 x 4096 x 4096 on the prefill GEMM, the others
+    on the kernel that splits K over waves), zero points U{0..15}. Primary check: against fp64 A . Wbf16^T with the dequantised weights
     rounded to bf16 once, as the kernel feeds them, within the output's bf16
     rounding plus fp32 accumulation. Secondary: against the oracle's exact
     dequantisation, plus the rigorous bound 2^-9 sum |a w| of that rounding."""
