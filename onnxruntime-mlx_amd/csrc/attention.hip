@@ -175,13 +175,22 @@ __device__ __forceinline__ void unpack8(u32x4_t w, float (&x)[8]) {
         x[2 * i + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(w[i] >> 16)));
     }
 }
+// Rounded to T, nearest even, by the hardware's conversions (two values at a time in bf16:
+// with integer arithmetic gqa_kv_rows took 2.75 us for 2 tokens of 8 heads of 128, 2.33 now).
 template <typename T>
 __device__ __forceinline__ u32x4_t pack8(const float (&x)[8]) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
     u32x4_t w;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        w[i] = (uint32_t)__builtin_bit_cast(uint16_t, from_f32<T>(x[2 * i])) |
-               (uint32_t)__builtin_bit_cast(uint16_t, from_f32<T>(x[2 * i + 1])) << 16;
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (std::is_same<T, half_t>::value) {
+            const half2_t v = {(half_t)x[2 * i], (half_t)x[2 * i + 1]};
+            w[i] = __builtin_bit_cast(uint32_t, v);
+        } else {
+            const bf16x2_t v = {(__bf16)x[2 * i], (__bf16)x[2 * i + 1]};
+            w[i] = __builtin_bit_cast(uint32_t, v);
+        }
+    }
     return w;
 }
 // Rotates the pieces w0 (dims c .. c + 7) and w1 (dims hd/2 + c ..) of a head whose rotary
