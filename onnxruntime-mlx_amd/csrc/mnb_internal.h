@@ -16,14 +16,15 @@ int mnb_blk(const T* A, const uint8_t* B, const T* S, const uint8_t* Z, T* Y, in
             int bs, hipStream_t st);
 
 // Shapes of 4-bit weights with fp16 or bf16 activations that take mnb_blk; larger ones take
-// the prefill GEMM's shared weight tiles. On MI355X, GEMM against mnb_blk in fp16: 8 rows of
-// 4096 x 14336 24.7 -> 12.6 us, 64 rows of 4096 x 4096 21.7 -> 10.4 us. Past 64 rows the GEMM
-// has too few tiles for the chip while M * N is below about 2^20: 128 rows of 8960 x 1536
-// 43.3 -> 16.6 us, 256 rows 44.1 -> 24.8 us, 128 rows of 4096 x 4096 21.4 -> 13.6 us; level
-// at 512 x 8960 x 1536 (46.0, 45.6 us) and at 384 x 4096 x 4096 (34.8, 34.1 us), and behind
-// at 512 x 4096 x 4096 (33.4, 40.4 us) and 1024 x 896 x 1152 (11.3, 13.3 us).
+// the prefill GEMM's shared weight tiles. Up to 32 rows the GEMM's tiles are mostly padding
+// (MI355X, GEMM against mnb_blk in fp16: 8 rows of 4096 x 14336 21.7 -> 11.7 us). Beyond,
+// mnb_blk gains while its tiles of 32 x 64 outputs all run at once, a CU to each: the GEMM has
+// a quarter of the tiles and leaves CUs idle (240 tiles, 96 rows of K 4096, N 5120: 1.5 times
+// as fast as the GEMM; 256 tiles, 512 rows of K 896 to 14336, N 1024: 1.2 to 1.7 times). From
+// 257 tiles on, each CU dequantises for two: 320 (128 rows of N 5120) 1.12 times at K 4096 but
+// 0.92 at K 8960, 448 (64 rows of N 14336) 0.75 to 0.97.
 inline bool mnb_takes_blk(int64_t M, int64_t N) {
-    return M <= 64 || (M <= 512 && M * N < (1 << 20));
+    return M <= 32 || (M <= 512 && ((M + 31) / 32) * ((N + 63) / 64) <= device_cu_count());
 }
 
 // The prefill GEMM (mnb_gemm.hip): bs in {32, 64, 128}, A and B 16-byte aligned,

@@ -51,6 +51,9 @@ def _run(ortmi, oracle, dt, M, K, N, bits, block, asym, edit=None):
     (65, 1536, 130, 4, 32, True),   # past 64 rows, too few outputs for the prefill GEMM
     (200, 896, 515, 4, 64, False),
     (512, 360, 1030, 4, 32, True),
+    (512, 360, 1000, 4, 32, True),  # 256 tiles of 32 x 64: a CU to each
+    (33, 896, 8192, 4, 128, False),
+    (33, 896, 8193, 4, 128, False), # and one column more, on the prefill GEMM
 ])
 def test_mnb_blk(ortmi, oracle, dt, M, K, N, bits, block, asym):
     got, A, W = _run(ortmi, oracle, dt, M, K, N, bits, block, asym)

@@ -249,8 +249,8 @@ def test_mnb_gemv_fp16_interleaved_symmetric(ortmi, oracle, K, N):
 @pytest.mark.parametrize("K,N,block", [(256, 192, 32), (512, 256, 64), (384, 160, 128),
                                        (1176, 64, 32)])
 def test_mnb_gemm_fp16(ortmi, oracle, M, K, N, block):
-    """Small fp16 products: all of them, being below 65 rows or 2^20 outputs, on the kernel
-    that splits K over waves (the prefill GEMM: test_mnb_gemm_forms)."""
+    """Small fp16 products, all of them on the kernel that splits K over waves (the prefill
+    GEMM: test_mnb_gemm_forms)."""
     rng = np.random.default_rng(M * 11 + K + N + block)
     A, B, s, zp = _mnb_inputs(rng, M, N, K, block, dtype=np.float16)
     got = host(ortmi.matmul_nbits(dev(A), dev(B), dev(s), dev(zp), K=K, N=N, block_size=block))
@@ -280,7 +280,7 @@ def _check_gemm_rows(oracle, got_rows, A_rows, B, s, zp, N, K, block, what):
 
 @pytest.mark.parametrize("M,N,K", [
     (512, 4096, 4096),   # the prefill GEMM config
-    (512, 1536, 8960),   # the decoder prefill's down_proj (K split over waves)
+    (512, 1536, 8960),   # the decoder prefill's down_proj (64x64 tiles, k split)
     (512, 2048, 1536),   # the decoder prefill's merged QKV
 ])
 def test_mnb_gemm_config2_shape(ortmi, oracle, M, N, K):
