@@ -13,7 +13,7 @@
 //    DPP row), adds the bias, and keeps an online softmax; the 16 team states are
 //    merged through LDS. Causal: query s attends keys [0, valid_past + s].
 //  - gqa_f32_tile_kernel: fp32 at head sizes 64, 96 and 128 without a bias, on the fp32
-//    matrix cores.
+//    matrix cores, where rows and keys are many enough (f32_tiles_pay).
 // The KV contract (shared buffer vs growing, attention.rs:636-651) is that of
 // ortmi_group_query_attention.
 //
@@ -540,6 +540,34 @@ __global__ __launch_bounds__(64 * kF32Waves, 1) void gqa_f32_tile_kernel(
     }
 }
 
+// Whether the tiles finish an fp32 call before a workgroup per query row does (head 64, 96 or
+// 128). Few keys or rows leave a tile's waves idle: 32 heads of 128 on 8, one token over 17
+// keys, 15.0 us against 10.3 with a workgroup per row; 33 tokens 26.5 and 15.7; 32 sequences
+// of one token over 91 keys, a KV head to each query head, 100 and 37; level at about 100
+// keys, and 300 tokens 73 and 155. The estimates are in us, fitted to 7800 calls on MI355X
+// (1-512 tokens, 1-32 sequences, up to 4500 keys, 8-32 heads); with the tiles favoured by
+// less than a fifth the rows keep the call, and of those calls 6 were slower on the chosen
+// kernel than a workgroup per row by more than 3 %, the worst 1.2 times.
+bool f32_tiles_pay(int64_t B, int64_t S, int64_t H, int64_t KV, int hd, int64_t vp) {
+    struct Cost {
+        double row0, row_key, row, pair;          // a workgroup per row
+        double tile0, round, round_key, tile_key;  // tiles
+        int per_cu;                                // tiles that share a CU (LDS)
+    };
+    const Cost c = hd == 64   ? Cost{7.1, .07, .0022, 3.4e-5, 0., 11., .018, 1.6e-4, 2}
+                   : hd == 96 ? Cost{7.7, .10, .0026, 4.7e-5, 3., 11.4, .052, 1.7e-4, 1}
+                              : Cost{8.2, .13, .0029, 6.2e-5, 3.9, 12.5, .072, 2.0e-4, 1};
+    const double n = (double)(vp + S), seen = (double)vp + 0.5 * (double)(S + 1);
+    const double rows = (double)(B * S * H);
+    const int64_t tiles = B * KV * ((S * (H / KV) + kF32Rows - 1) / kF32Rows);
+    const int64_t slots = (int64_t)device_cu_count() * c.per_cu;
+    const double rounds = (double)((tiles + slots - 1) / slots);
+    double tile = c.tile0 + rounds * (c.round + c.round_key * n) + c.tile_key * tiles * seen;
+    // Two or three waves with keys that are hidden to some rows, at heads of 96 and 128.
+    if (hd > 64 && S > 1 && n > 32 && n <= 96) tile += 6.;
+    return 1.2 * tile < c.row0 + c.row_key * n + c.row * rows + c.pair * rows * seen;
+}
+
 template <typename T>
 int run_gqa_ex(const void* query, const void* key, const void* value, const void* past_key,
                const void* past_value, int64_t cap, int total, const void* cos_c,
@@ -590,7 +618,7 @@ int run_gqa_ex(const void* query, const void* key, const void* value, const void
         const int64_t tiles = ((int64_t)S * (H / KV) + kF32Rows - 1) / kF32Rows;
         const int64_t grid = (int64_t)B * KV * tiles;
         if (!bias && a16(ws) && a16(pk) && (hd == 64 || hd == 96 || hd == 128) &&
-            grid <= 0x7fffffffLL) {
+            grid <= 0x7fffffffLL && f32_tiles_pay(B, S, H, KV, hd, vp)) {
             auto launch = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * kF32Waves), 0, st, qf,
                                    static_cast<const float*>(pk), static_cast<const float*>(pv),

@@ -129,7 +129,7 @@ def test_gqa_tile_options(ortmi, dt, hd, opt):
 @pytest.mark.parametrize("hd", [64, 96, 128])
 def test_gqa_f32_tile_options(ortmi, hd, opt):
     """fp32: the sign branch, and the fallback for rows that are not 16-byte aligned."""
-    check(ortmi, "f32", 2, 37, 70, 8, 2, hd, **opt)
+    check(ortmi, "f32", 2, 130, 150, 8, 2, hd, **opt)
 
 
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
@@ -184,6 +184,34 @@ def test_gqa_f32_tile_infinite_value_stays_in_its_rows(ortmi):
     out = out.cpu()[0]
     assert torch.isfinite(out[:20]).all() and (out[20:, 3] == math.inf).all()
     out[20:, 3] = 0
+    assert torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("hd", [64, 96, 128])
+@pytest.mark.parametrize("B,S,past,H,KV", [
+    (1, 1, 16, 32, 8), (1, 17, 0, 14, 2), (2, 33, 16, 8, 8),    # few keys
+    (32, 1, 90, 16, 16),                                        # one row to a tile
+    (1, 60, 40, 32, 8), (1, 100, 0, 24, 8), (4, 9, 100, 32, 8),  # to both sides of the line
+    (1, 257, 0, 8, 2),
+])
+def test_gqa_f32_few_keys(ortmi, hd, B, S, past, H, KV):
+    """fp32 calls on both sides of the rule that chooses tiles or a workgroup per row."""
+    check(ortmi, "f32", B, S, past, H, KV, hd)
+
+
+@pytest.mark.parametrize("hd,at", [(64, 130), (96, 201), (128, 255)])
+def test_gqa_f32_tile_infinite_value(ortmi, hd, at):
+    """As above, with keys enough for the tiles."""
+    S, H = 257, 8
+    g = torch.Generator().manual_seed(6)
+    q, k, v = (torch.randn((1, S, H * hd), generator=g) for _ in range(3))
+    v[0, at, 3] = math.inf
+    z = torch.zeros((1, H, 0, hd), device="cuda")
+    out, _, _ = ortmi.group_query_attention(q.cuda(), k.cuda(), v.cuda(), z, z, None, S, None, None,
+                                            num_heads=H, kv_num_heads=H)
+    out = out.cpu()[0]
+    assert torch.isfinite(out[:at]).all() and (out[at:, 3] == math.inf).all()
+    out[at:, 3] = 0
     assert torch.isfinite(out).all()
 
 
