@@ -1760,6 +1760,15 @@ __global__ __launch_bounds__(64 * kMergeRows) void paged_merge_kernel(
     const int ns = min(nsplit, nsplit_row[r]);  // at most 64 (the callers' split rules)
     if (ns <= 0) return;
     const float* p = part + r * nsplit * (vhd + 2);
+    // The first 8 splits of the first 128 dims, requested with the states that weigh them.
+    auto fetch = [&](float2 (&v)[8], int i0, int d) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            v[i] = *reinterpret_cast<const float2*>(p + min(i0 + i, ns - 1) * (vhd + 2) +
+                                                    min(d, vhd - 2));
+    };
+    float2 v[8];
+    fetch(v, 0, 2 * lane);
     const bool mine = lane < ns;
     const float m = mine ? p[lane * (vhd + 2) + vhd] : -INFINITY;
     const float lp = mine ? p[lane * (vhd + 2) + vhd + 1] : 0.f;
@@ -1768,13 +1777,11 @@ __global__ __launch_bounds__(64 * kMergeRows) void paged_merge_kernel(
     const float w = m != -INFINITY ? __expf(m - M) : 0.f;
     const float L = wave_sum(w * lp) + (sk != -INFINITY ? __expf(sk - M) : 0.f);
     const float inv = L > 0.f ? 1.0f / L : 0.f;
-    for (int d = 2 * lane; d < vhd; d += 128) {
+    for (int d0 = 0; d0 < vhd; d0 += 128) {
+        const int d = d0 + 2 * lane;
         float a = 0.f, b = 0.f;
         for (int i0 = 0; i0 < ns; i0 += 8) {
-            float2 v[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                v[i] = *reinterpret_cast<const float2*>(p + min(i0 + i, ns - 1) * (vhd + 2) + d);
+            if (d0 + i0 > 0) fetch(v, i0, d);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const float wi = __shfl(w, i0 + i, 64);  // 0 past the last split
@@ -1782,6 +1789,7 @@ __global__ __launch_bounds__(64 * kMergeRows) void paged_merge_kernel(
                 b = wi != 0.f ? fmaf(v[i].y, wi, b) : b;
             }
         }
+        if (d >= vhd) continue;
         T* o = out + r * vhd + d;
         o[0] = from_f32<T>(a * inv);
         o[1] = from_f32<T>(b * inv);
