@@ -1434,6 +1434,17 @@ __global__ __launch_bounds__(256) void paged_rows_kernel(
     auto store = [](T* p, u32x4_t w) { *reinterpret_cast<u32x4_t*>(p) = w; };
     const T* src = is_q ? q + row : k + row;
     u32x4_t w0 = load(src), w1 = load(src + half);
+    // The slot of a key row: its lookup goes out with the rotary entries'.
+    int64_t slot = -1;
+    if (!is_q) {
+        if (slot_mapping) {
+            slot = slot_mapping[tok];
+        } else {
+            const int lb = pos / blk;
+            const int phys = lb < maxb ? bt[(int64_t)b * maxb + lb] : -1;
+            slot = phys < 0 ? -1 : (int64_t)phys * blk + pos % blk;
+        }
+    }
     if (cos_c) {
         // A position outside the cache violates the op contract; clamp the row so the read
         // stays inside the cos/sin tensors.
@@ -1447,14 +1458,6 @@ __global__ __launch_bounds__(256) void paged_rows_kernel(
     }
     store(knew + row, w0);
     store(knew + row + half, w1);
-    int64_t slot;
-    if (slot_mapping) {
-        slot = slot_mapping[tok];
-    } else {
-        const int lb = pos / blk;
-        const int phys = lb < maxb ? bt[(int64_t)b * maxb + lb] : -1;
-        slot = phys < 0 ? -1 : (int64_t)phys * blk + pos % blk;
-    }
     if (slot < 0 || slot >= nblk * blk) return;
     const int64_t dst = (slot * KV + kvh) * hd + c;
     store(kcache + dst, w0);
