@@ -2666,10 +2666,16 @@ static int run_paged(const void* query, const void* key, const void* value, void
     // for, and the pair finished no sooner than in sequence. Groups of 3 query heads left
     // their single tokens to the tiles before (32 sequences to 6000 keys, 24 / 8 heads of
     // 128: 240 -> 136 us). Groups of 6 and 7 gain nothing: a workgroup's instructions bind it
-    // (24 sequences, 12 / 2 heads of 128: 105 us, 124 here).
+    // (24 sequences, 12 / 2 heads of 128: 105 us, 124 here). Single tokens of groups of 3 also
+    // stay with tiles that prompt chunks need in any case, while those run nearly all at once:
+    // up to two for a CU by this bound, which takes every sequence for the longest (19
+    // sequences to 789 keys, one with 3 new tokens: 37 us, 52 with this kernel before the
+    // tiles; 8 new tokens alone 31 and 33; from 2.06 to a CU on 0.98 to 1.44 times as fast with
+    // it, and where single tokens are all, 1.1 to 1.7 times at any number).
     bool dec = false;
     if constexpr (VHD == HD) {
-        dec = vcache && value && pow2 && (G == 1 || G == 2 || G == 3 || G == 4 || G == 8);
+        const bool three = G == 3 && (T_ == batch || (int64_t)mt * KV * ns > 2 * device_cu_count());
+        dec = vcache && value && pow2 && (G == 1 || G == 2 || three || G == 4 || G == 8);
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(mt, KV, ns), dim3(256), 0, st, tiles, count, cum,
                                past, pk, blk_shift, qrot, H, sc, sink ? sink32 : nullptr, chunk,

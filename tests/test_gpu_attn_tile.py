@@ -302,6 +302,14 @@ def test_paged_group_sizes(ortmi, oracle, H, KV, d, new_max, interleaved):
                rope=True, interleaved=interleaved)
 
 
+@pytest.mark.parametrize("batch,maxb", [(4, 40), (26, 70)])
+def test_paged_groups_of_three_beside_chunks(ortmi, oracle, batch, maxb):
+    """Single tokens of 3 query heads per KV head beside chunks: on the tiles where those all
+    run at once, on the decode kernel where they do not (26 sequences, 3 splits)."""
+    _run_paged(ortmi, oracle, 24, 8, 64, nb=maxb * batch, blk=16, batch=batch, seed=batch,
+               new_max=2, rope=True)
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("hd,H,KV", [(64, 8, 8), (96, 6, 2), (128, 8, 1)])
 @pytest.mark.parametrize("shared", [True, False])
