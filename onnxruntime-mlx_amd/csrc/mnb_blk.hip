@@ -15,9 +15,9 @@
 //
 // Bound: the weight stream and, from about 16 rows, the dequantisation (about 17
 // vector instructions per 8 codes). Measured on MI355X, before (VALU tile product, or
-// the prefill GEMM's tiles for 4-bit fp16) and now: one row of 3072 x 32064 8-bit 501
-// -> 24.8 us (4.0 TB/s), 8 rows of 4096 x 14336 4-bit 24.7 -> 12.6 us (2.3 TB/s), 512
-// x 896 x 1152 fp32 185 -> 15.8 us, 512 x 4096 x 4096 fp32 866 -> 103 us.
+// the prefill GEMM's tiles for 4-bit fp16) and now: one row of 3072 x 32064 8-bit 497
+// -> 23.6 us (4.4 TB/s), 8 rows of 4096 x 14336 4-bit 21.7 -> 11.5 us (2.9 TB/s), 512
+// x 896 x 1152 fp32 185 -> 14.8 us, 512 x 4096 x 4096 fp32 866 -> 98 us.
 #include <algorithm>
 
 #include "common.h"
