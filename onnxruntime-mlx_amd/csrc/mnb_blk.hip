@@ -51,7 +51,8 @@ constexpr bool blk_scaled() { return sizeof(T) == 2 && BITS == 4; }
 
 // A code enters bf16 operands as (q - zp) times this power of two (exact), so that a
 // chunk's 32 products sum to no more than the largest activation: no overflow that
-// the scaled weights would not have had. fp16 sums cannot overflow fp32.
+// the scaled weights would not have had. The sums stay in this unit to the end, where
+// the scale of no block can overflow either. fp16 sums cannot overflow fp32.
 template <typename T, int BITS, bool SC>
 constexpr float blk_unit() {
     if (std::is_same<T, half_t>::value || SC) return 1.f;
@@ -77,8 +78,8 @@ __device__ __forceinline__ uint32_t high_halves(float lo, float hi) {
 // 8 codes of 4 bits as 8 weights (q - zp) * s rounded once to T. fp16 comes in pair
 // order (0,4) (1,5) (2,6) (3,7), the activations permuted alike: (1024 + q) -
 // (1024 + zp) is exact, the product rounds. bf16 comes in order: a byte 0000qqqq read
-// as fp8 (e4m3) is q * 2^-9 exactly, and both products of the fused multiply-add are
-// exact in fp32, so only the conversion rounds.
+// as fp8 (e4m3) is q * 2^-9 exactly, the convert's scale makes it q, and both products of
+// the fused multiply-add are exact in fp32, so only the conversion rounds.
 template <typename T>
 __device__ __forceinline__ u32x4_t scaled_codes(uint32_t w, uint32_t zp, uint32_t sbits,
                                                 uint32_t magic) {
@@ -93,14 +94,14 @@ __device__ __forceinline__ u32x4_t scaled_codes(uint32_t w, uint32_t zp, uint32_
             r[j] = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(half2_t, m) - z2) * s2);
         }
     } else {
-        const float s = to_f32((uint16_t)sbits) * 512.f, zo = -(float)zp * (1.f / 512.f) * s;
+        const float s = to_f32((uint16_t)sbits), zo = -(float)zp * s;
         const uint32_t ev = w & 0x0F0F0F0Fu, od = (w >> 4) & 0x0F0F0F0Fu;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const auto e = h ? __builtin_amdgcn_cvt_pk_f32_fp8((int)ev, true)
-                             : __builtin_amdgcn_cvt_pk_f32_fp8((int)ev, false);
-            const auto o = h ? __builtin_amdgcn_cvt_pk_f32_fp8((int)od, true)
-                             : __builtin_amdgcn_cvt_pk_f32_fp8((int)od, false);
+            const auto e = h ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)ev, 512.f, true)
+                             : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)ev, 512.f, false);
+            const auto o = h ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)od, 512.f, true)
+                             : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)od, 512.f, false);
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const bf16x2_t v = {(__bf16)fmaf(e[i], s, zo), (__bf16)fmaf(o[i], s, zo)};
@@ -494,14 +495,13 @@ __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
 #pragma unroll
                     for (int i = 0; i < MT; ++i) acc[i][t] = blk_mfma<T>(ao[i][0], bo, acc[i][t]);
                 } else {
-                    constexpr float inv = 1.f / blk_unit<T, BITS, SC>();
                     float sc;
                     if constexpr (sizeof(T) == 4)
-                        sc = __uint_as_float(sv[t][c]) * inv;
+                        sc = __uint_as_float(sv[t][c]);
                     else if constexpr (std::is_same<T, half_t>::value)
                         sc = (float)__builtin_bit_cast(half_t, (uint16_t)(sv[t][c] & 0xffffu));
                     else
-                        sc = to_f32((uint16_t)(sv[t][c] & 0xffffu)) * inv;
+                        sc = to_f32((uint16_t)(sv[t][c] & 0xffffu));
                     constexpr int W = BITS / 4;  // words per chunk and lane
                     const u32x4_t bo =
                         blk_codes<T, BITS>(w[t][W * c], w[t][W * c + W - 1], zv[t][c]);
@@ -563,6 +563,7 @@ __global__ __launch_bounds__(64 * NW, 2) void mnb_blk_kernel(
         float v = 0.f;
 #pragma unroll
         for (int j = 0; j < NW; ++j) v += red[((j * MT * NT + it) * 4 + e) * 64 + lane];
+        v *= 1.f / blk_unit<T, BITS, SC>();
         const int m = m0 + 16 * (it / NT) + 4 * g + e, n = n0 + 16 * (it % NT) + li;
         if constexpr (sizeof(T) == 4) {
             // A NaN whose payload lies in the low 16 bits alone entered as an infinity (its

@@ -30,24 +30,24 @@ __device__ __forceinline__ uint4 dequant_word_pairs(uint32_t w, half2_t zoff, ha
 
 
 // bf16 weights, in the codes' own order (the activations then need no permutation): a byte
-// 0000qqqq read as fp8 (e4m3) is q * 2^-9 exactly, and q * s - zp * s is exact in fp32 (s has
-// 8 mantissa bits), so that only the conversion rounds: bf16((q - zp) * s). 19 vector
-// instructions per 8 codes; by way of fp16 pairs, widened and scaled in fp32, 32 (1999 x
+// 0000qqqq read as fp8 (e4m3) is q * 2^-9 exactly, the convert's scale makes it q, and q * s -
+// zp * s is exact in fp32 (s has 8 mantissa bits), so that only the conversion rounds:
+// bf16((q - zp) * s). 19 vector instructions per 8 codes; by way of fp16 pairs, widened and scaled in fp32, 32 (1999 x
 // 17920 x 1536, block 128: 159 us, 143 us now).
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ uint4 dequant_word_bf16(uint32_t w, float s512, float zs) {
+__device__ __forceinline__ uint4 dequant_word_bf16(uint32_t w, float s, float zs) {
     const uint32_t ev = w & 0x0F0F0F0Fu, od = (w >> 4) & 0x0F0F0F0Fu;
     uint32_t r[4];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const auto e = h ? __builtin_amdgcn_cvt_pk_f32_fp8((int)ev, true)
-                         : __builtin_amdgcn_cvt_pk_f32_fp8((int)ev, false);
-        const auto o = h ? __builtin_amdgcn_cvt_pk_f32_fp8((int)od, true)
-                         : __builtin_amdgcn_cvt_pk_f32_fp8((int)od, false);
+        const auto e = h ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)ev, 512.f, true)
+                         : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)ev, 512.f, false);
+        const auto o = h ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)od, 512.f, true)
+                         : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)od, 512.f, false);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const bf16x2_t v = {(__bf16)fmaf(e[i], s512, zs), (__bf16)fmaf(o[i], s512, zs)};
+            const bf16x2_t v = {(__bf16)fmaf(e[i], s, zs), (__bf16)fmaf(o[i], s, zs)};
             r[2 * h + i] = __builtin_bit_cast(uint32_t, v);
         }
     }
@@ -60,7 +60,7 @@ __device__ __forceinline__ uint4 dequant_word_bf16(uint32_t w, float s512, float
 template <typename T>
 struct GemmDq {
     half2_t zoff, s2;  // fp16: 1024 + zero point and the scale, as pairs
-    float s512, zs;    // bf16: 512 * scale, -zero point * scale
+    float s, zs;       // bf16: scale, -zero point * scale
 };
 template <typename T>
 __device__ __forceinline__ GemmDq<T> gemm_dq(float zf, uint16_t sbits) {
@@ -70,7 +70,7 @@ __device__ __forceinline__ GemmDq<T> gemm_dq(float zf, uint16_t sbits) {
         d.zoff = half2_t{(half_t)(1024.f + zf), (half_t)(1024.f + zf)};
         d.s2 = half2_t{sh, sh};
     } else {
-        d.s512 = to_f32(sbits) * 512.f;
+        d.s = to_f32(sbits);
         d.zs = -zf * to_f32(sbits);
     }
     return d;
@@ -78,7 +78,7 @@ __device__ __forceinline__ GemmDq<T> gemm_dq(float zf, uint16_t sbits) {
 template <typename T>
 __device__ __forceinline__ uint4 gemm_dequant(uint32_t w, const GemmDq<T>& d) {
     if constexpr (std::is_same<T, half_t>::value) return dequant_word_pairs(w, d.zoff, d.s2);
-    else return dequant_word_bf16(w, d.s512, d.zs);
+    else return dequant_word_bf16(w, d.s, d.zs);
 }
 template <typename T>
 __device__ __forceinline__ float16_t gemm_mfma(half8_t a, half8_t b, float16_t c) {

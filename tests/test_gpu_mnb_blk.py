@@ -128,6 +128,30 @@ def test_mnb_blk_one_row_keeps_weights(ortmi, oracle, dt, K, N, block, asym):
     assert (np.abs(got - exact) <= bound).all()
 
 
+@pytest.mark.parametrize("dt,M,N,bits", [
+    ("bf16", 40, 96, 4), ("bf16", 600, 2048, 4), ("bf16", 3, 96, 8), ("f32", 20, 96, 4),
+    ("f32", 20, 96, 8)])
+def test_mnb_large_scales(ortmi, oracle, dt, M, N, bits):
+    """Scales near the largest the type holds, activations that keep the sums finite: each
+    form's weights (q - zp) * s are finite, and so are its products."""
+    import torch
+
+    K, tdt = 256, {"bf16": torch.bfloat16, "f32": torch.float32}[dt]
+    rng = np.random.default_rng(M + bits)
+    A, B, s, zp = _mnb_inputs(rng, M, N, K, 32, bits=bits)
+    top = 2.0 ** (123 if bits == 4 else 119)  # * 15 or 255 < 2^127
+    s = s / s.max() * top
+    dA, ds = dev(A * 2.0 ** -20, tdt), dev(s, tdt)
+    got = host(ortmi.matmul_nbits(dA, dev(B), ds, dev(zp), K=K, N=N, bits=bits, block_size=32))
+    A, s = dA.double().cpu().numpy(), ds.float().cpu().numpy()
+    W = oracle.mnb_dequant(B, s, zp, N, K, bits, 32).astype(np.float64)
+    want, mag = A @ W.T, np.abs(A) @ np.abs(W).T
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    # Weights rounded to bf16 at 4 bits: one rounding of each product.
+    u = 2.0 ** -8 if dt == "bf16" and bits == 4 else 2.0 ** -16
+    assert (np.abs(got - want) <= u * mag + (2.0 ** -8 if dt == "bf16" else 0) * np.abs(want)).all()
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 def test_mnb_blk_fp32_signalling_nan(ortmi, oracle, bits):
     """A NaN whose payload lies in the low 16 bits alone gives NaN rows, not infinities."""
